@@ -116,29 +116,108 @@ int check_fluence(const char *fn, const xo_fluence &f, uint64_t det_end, uint64_
     return 0;
 }
 
-/* The LDS fluence box of a voxel run: kFlBox bins of a Cartesian grid
- * around the point where the source enters it (centred in x and y,
- * starting at that depth), clamped into the grid; off for other grids, or
- * when the grid or the LDS budget is too small. */
-void place_fluence_box(const xo_mcvox_cfg &cfg, McvoxParams &P) {
-    P.fl_box_on = 0;
-    const xo_fluence &F = cfg.fluence;
-    if (F.enabled != XO_FLUENCE_XYZ || F.shape[0] < (uint32_t)kFlBoxX ||
-        F.shape[1] < (uint32_t)kFlBoxY || F.shape[2] < (uint32_t)kFlBoxZ ||
-        mcvox_lds_bytes(P) > 32768u)
-        return;
-    const float *sp = cfg.source_kind == XO_SRC_LINE ? cfg.line.position : cfg.gaussian.position;
-    const int32_t ext[3] = {kFlBoxX, kFlBoxY, kFlBoxZ};
-    const int32_t back[3] = {kFlBoxX / 2, kFlBoxY / 2, 0};
+/* The window of at most `budget` fluence bins held in LDS: the whole grid if
+ * it fits, else a box around the point where the source enters it, twice as
+ * wide (x, y) as deep, or as wide (r) as deep, starting at that depth. */
+FluenceL fluence_window(const xo_fluence &F, const float src[3], uint32_t budget) {
+    FluenceL W = fluence_to_device(F);
+    if (F.enabled == XO_FLUENCE_NONE || budget < 64u) return W;
+    const bool rz = F.enabled == XO_FLUENCE_RZ;
+    const uint32_t shape[3] = {F.shape[0], rz ? 1u : F.shape[1], F.shape[2]};
+    double step[3], at[3];
     for (int k = 0; k < 3; ++k) {
-        const double f = ((double)sp[k] - F.top_left[k]) * F.inv_step[k];
-        int64_t c = std::isfinite(f) ? (int64_t)std::floor(f) - back[k] : 0;
-        const int64_t hi = (int64_t)F.shape[k] - ext[k];
-        c = c < 0 ? 0 : (c > hi ? hi : c);
-        P.fl_box[k] = (int32_t)c;
+        step[k] = F.inv_step[k] > 0.0f && std::isfinite(F.inv_step[k])
+                      ? 1.0 / (double)F.inv_step[k] : 1.0;
+        at[k] = (double)src[k] - F.top_left[k];
     }
-    P.fl_box_on = 1;
+    if (rz) at[0] = std::sqrt(at[0] * at[0] + at[1] * at[1]);
+    /* extents of edge e, 2 e (or e for r) and e / 2 (e for r): the largest e
+     * within the budget, by bisection of its logarithm */
+    const double wide[3] = {1.0, 1.0, rz ? 1.0 : 0.5};
+    auto extents = [&](double e, uint32_t ext[3]) {
+        double n = 1.0;
+        for (int k = 0; k < 3; ++k) {
+            const double v = std::floor(e * wide[k] / step[k]);
+            ext[k] = v < 1.0 ? 1u : (v > (double)shape[k] ? shape[k] : (uint32_t)v);
+            n *= ext[k];
+        }
+        return n;
+    };
+    double lo = std::log(1e-30), hi = std::log(1e30);
+    for (int it = 0; it < 60; ++it) {
+        const double mid = 0.5 * (lo + hi);
+        (extents(std::exp(mid), W.ext) <= (double)budget ? lo : hi) = mid;
+    }
+    if (extents(std::exp(lo), W.ext) > (double)budget) return W;
+    for (int k = 0; k < 3; ++k) {
+        const double f = at[k] / step[k] - ((k == 2) ? 0.0 : 0.5 * W.ext[k]);
+        const double top = (double)(shape[k] - W.ext[k]);
+        W.origin[k] = !(f > 0.0) ? 0u : (f > top ? (uint32_t)top : (uint32_t)f);
+    }
+    W.bins = W.ext[0] * W.ext[1] * W.ext[2];
+    return W;
 }
+
+/* Threads per block, fluence window and grid of a single-simulation launch of
+ * P.lanes lanes. `waves`: the waves per SIMD its registers allow, fewer for a
+ * small run. Without a fluence grid: blocks of XO_BLOCK. With one, windows
+ * share the CU's LDS, so a CU takes one block of up to four waves per SIMD
+ * or two of up to four each, in whole waves per SIMD (blocks of 896 threads,
+ * 3.5 waves, measured 10.8 ms where 768 take 9.5: the second block's extra
+ * waves land on SIMDs that are full). 6e6 packets into an 8000-bin r-z grid,
+ * hardware arithmetic: 176 ms with every deposit in memory, 26 ms with 2025
+ * bins in seven blocks of 256, 18.5 with 4096 in four of 384, 9.5 with all
+ * 8000 in two of 768. A lane count that the caller left open (`open`) is cut
+ * to what is resident. */
+template <class Params, class Fit>
+static int shape_launch(xo_ctx *ctx, const xo_fluence &F, const float src[3], int waves,
+                        bool open, Params &P, uint32_t *block, uint32_t *blocks,
+                        const Fit &fit) {
+    *block = XO_BLOCK;
+    P.fluence = fluence_to_device(F);
+    if (F.enabled != XO_FLUENCE_NONE) {
+        const size_t fixed = fit.lds(P) + 1024u; /* and the static LDS */
+        for (; waves >= 1; --waves) {
+            if (waves > 4 && (waves & 1)) continue;
+            const uint32_t per_cu = waves > 4 ? 2u : 1u;
+            const uint32_t threads = XO_BLOCK * (uint32_t)waves / per_cu;
+            const size_t share = ctx->lds_per_cu / per_cu;
+            const uint32_t budget = share > fixed ? (uint32_t)((share - fixed) / 8u) : 0u;
+            Params Q = P;
+            /* a bin pays where a block adds to it more than once: four bins
+             * per packet of a block at most (1e5 voxel packets on 256
+             * blocks: 4.11 ms without a window, 4.22 with 4000 bins, 4.29
+             * with 7500; 3e5 layered ones: 9.29, 8.31, 8.26) */
+            const uint64_t grid = (P.lanes + threads - 1) / threads;
+            const uint64_t useful = 4u * (P.npackets / grid);
+            Q.fluence = fluence_window(
+                F, src,
+                (uint32_t)std::min<uint64_t>(std::min(budget, kFluenceWindowMax), useful));
+            int n = 0;
+            XO_HIP(fit.occupancy(Q, threads, &n));
+            if (n < (int)per_cu) continue;
+            P.fluence = Q.fluence;
+            *block = threads;
+            if (open) P.lanes = std::min(P.lanes, per_cu * threads * ctx->cus);
+            break;
+        }
+    }
+    *blocks = (P.lanes + *block - 1) / *block;
+    return 0;
+}
+
+struct FitMcml {
+    size_t lds(const McmlParams &P) const { return mcml_lds_bytes(P); }
+    hipError_t occupancy(const McmlParams &P, uint32_t block, int *n) const {
+        return occupancy_mcml(P, block, n);
+    }
+};
+struct FitMcvox {
+    size_t lds(const McvoxParams &P) const { return mcvox_lds_bytes(P); }
+    hipError_t occupancy(const McvoxParams &P, uint32_t block, int *n) const {
+        return occupancy_mcvox(P, block, n);
+    }
+};
 
 int check_pf(int pf_kind, const xo_pf &pf, uint32_t nlut, const char *what, uint32_t idx) {
     if (pf_kind == XO_PF_LUT) {
@@ -192,6 +271,33 @@ uint32_t choose_lanes(xo_ctx *ctx, uint32_t requested, int blocks_per_cu, uint64
     }
     if (lanes > ctx->max_lanes) lanes = ctx->max_lanes;
     return lanes;
+}
+
+/* Resident blocks of XO_BLOCK threads per CU that a static-schedule run's
+ * default lane count stands for. Its result is a function of the lane count,
+ * so the count follows from the configuration alone and not from what the
+ * compiled kernel's registers happen to allow: `waves` (7 for the layered
+ * kernel and the hardware arithmetic of the voxel one, 5 for its exact
+ * arithmetic) or what `lds` bytes per block leave of the CU's LDS. */
+static int static_blocks_per_cu(const xo_ctx *ctx, int waves, size_t lds) {
+    const int fit = (int)(ctx->lds_per_cu / (lds ? lds : 1u));
+    return fit < waves ? fit : waves;
+}
+
+/* The 16 KiB per block of a voxel run with a Cartesian grid that counted
+ * against the CU's LDS when the static default lane count was fixed. */
+static size_t static_box_bytes(const xo_mcvox_cfg &cfg, size_t lds) {
+    const xo_fluence &F = cfg.fluence;
+    return F.enabled == XO_FLUENCE_XYZ && F.shape[0] >= 16u && F.shape[1] >= 16u &&
+                   F.shape[2] >= 8u && lds <= 32768u
+               ? 16384u : 0u;
+}
+
+/* Waves per SIMD of a grid of `lanes`, at most `most`. */
+static int waves_per_simd(const xo_ctx *ctx, uint32_t lanes, int most) {
+    const uint32_t one = ctx->cus * XO_BLOCK;
+    const int n = (int)((lanes + one - 1) / one);
+    return n < most ? n : most;
 }
 
 uint64_t brick_bytes(const int32_t shape[3]) {
@@ -438,6 +544,7 @@ xo_ctx *xo_ctx_create(int device, uint32_t max_lanes, uint64_t xinit) {
     if ((e = hipGetDeviceProperties(&prop, device)) != hipSuccess)
         return fail("hipGetDeviceProperties", e);
     ctx->cus = (uint32_t)prop.multiProcessorCount;
+    ctx->lds_per_cu = (uint32_t)prop.maxSharedMemoryPerMultiProcessor;
     if ((e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking)) != hipSuccess)
         return fail("hipStreamCreate", e);
     if ((e = hipEventCreate(&ctx->ev0)) != hipSuccess) return fail("hipEventCreate", e);
@@ -488,7 +595,10 @@ int xo_ctx_info(xo_ctx *ctx, uint32_t *persistent_lanes, uint32_t *max_lanes,
     }
     int bpc = 1;
     XO_HIP(hipSetDevice(ctx->device));
-    XO_HIP(xo::occupancy_mcml(XO_PF_HG, XO_MAX_LAYERS * 64 + 8 * 102, false, &bpc));
+    xo::McmlParams P;
+    std::memset(&P, 0, sizeof(P));
+    P.lds_bins = 102;
+    XO_HIP(xo::occupancy_mcml(P, XO_BLOCK, &bpc));
     if (persistent_lanes) *persistent_lanes = choose_lanes(ctx, 0, bpc, ~0ull);
     if (max_lanes) *max_lanes = ctx->max_lanes;
     if (compute_units) *compute_units = ctx->cus;
@@ -650,15 +760,28 @@ static int mcml_run(xo_ctx *ctx, const xo_mcml_cfg *cfg, const float *lut, uint3
     P.accum = ctx->accum;
     P.npackets = npackets;
     P.flags = flags;
-    P.lds_bins = (!(flags & XO_FLAG_NO_LDS_BINS) && naccum <= XO_LDS_BINS_MAX)
-                     ? (uint32_t)naccum
-                     : 0u;
     P.lds_lut = (nlut && nlut <= XO_LDS_LUT_MAX) ? nlut : 0u;
     int bpc = 1;
-    XO_HIP(xo::occupancy_mcml(cfg->pf_kind, xo::mcml_lds_bytes(P),
-                                (flags & XO_FLAG_FAST_MATH) != 0, &bpc));
+    if (flags & XO_FLAG_STATIC_SCHEDULE) {
+        const bool small = !(flags & XO_FLAG_NO_LDS_BINS) && naccum <= XO_LDS_BINS_MAX;
+        bpc = xo::static_blocks_per_cu(ctx, 7, xo::mcml_lds_bytes(P) + 416u +
+                                                   (small ? 8u * naccum : 0u));
+    }
+    P.lds_bins = (!(flags & XO_FLAG_NO_LDS_BINS) && det_end <= XO_LDS_BINS_MAX)
+                     ? (uint32_t)det_end
+                     : 0u;
+    int waves = 1;
+    XO_HIP(xo::occupancy_mcml(P, XO_BLOCK, &waves));
+    if (!(flags & XO_FLAG_STATIC_SCHEDULE)) bpc = waves;
     P.lanes = choose_lanes(ctx, lanes, bpc, npackets);
-    uint32_t blocks = (P.lanes + XO_BLOCK - 1) / XO_BLOCK;
+    uint32_t block = 0, blocks = 0;
+    if (xo::shape_launch(ctx, cfg->fluence,
+                         cfg->source_kind == XO_SRC_LINE ? cfg->source.position
+                                                         : cfg->fiber.position,
+                         xo::waves_per_simd(ctx, P.lanes, waves),
+                         lanes == 0 && !(flags & XO_FLAG_STATIC_SCHEDULE), P, &block, &blocks,
+                         xo::FitMcml{}))
+        return -1;
 
     if (nlut)
         XO_HIP(hipMemcpyAsync(ctx->lut, lut, (size_t)nlut * 4, hipMemcpyHostToDevice,
@@ -667,7 +790,7 @@ static int mcml_run(xo_ctx *ctx, const xo_mcml_cfg *cfg, const float *lut, uint3
     XO_HIP(hipMemsetAsync(ctx->counters, 0, sizeof(unsigned long long) * (1 + XO_STAT_COUNT),
                           ctx->stream));
     XO_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-    if (npackets > 0) XO_HIP(xo::launch_mcml(P, blocks, ctx->stream));
+    if (npackets > 0) XO_HIP(xo::launch_mcml(P, blocks, block, ctx->stream));
     XO_HIP(hipEventRecord(ctx->ev1, ctx->stream));
     unsigned long long stats[1 + XO_STAT_COUNT];
     XO_HIP(hipMemcpyAsync(accum, ctx->accum, naccum * 8, hipMemcpyDeviceToHost, ctx->stream));
@@ -815,12 +938,24 @@ static int mcvox_run(xo_ctx *ctx, const xo_mcvox_cfg *cfg, const int32_t *voxels
                      ? (uint32_t)det_end
                      : 0u;
     P.lds_lut = (nlut && nlut <= XO_LDS_LUT_MAX) ? nlut : 0u;
-    xo::place_fluence_box(*cfg, P);
-    int bpc = 1;
-    XO_HIP(xo::occupancy_mcvox(cfg->pf_kind, xo::mcvox_lds_bytes(P),
-                                 (flags & XO_FLAG_FAST_MATH) != 0, &bpc));
+    int waves = 1;
+    XO_HIP(xo::occupancy_mcvox(P, XO_BLOCK, &waves));
+    int bpc = waves;
+    if (flags & XO_FLAG_STATIC_SCHEDULE) {
+        const bool fast = (flags & XO_FLAG_FAST_MATH) != 0;
+        bpc = xo::static_blocks_per_cu(ctx, fast ? 7 : 5,
+                                       xo::mcvox_lds_bytes(P) + 400u +
+                                           xo::static_box_bytes(*cfg, xo::mcvox_lds_bytes(P)));
+    }
     P.lanes = choose_lanes(ctx, lanes, bpc, npackets);
-    uint32_t blocks = (P.lanes + XO_BLOCK - 1) / XO_BLOCK;
+    uint32_t block = 0, blocks = 0;
+    if (xo::shape_launch(ctx, cfg->fluence,
+                         cfg->source_kind == XO_SRC_LINE ? cfg->line.position
+                                                         : cfg->gaussian.position,
+                         xo::waves_per_simd(ctx, P.lanes, waves),
+                         lanes == 0 && !(flags & XO_FLAG_STATIC_SCHEDULE), P, &block, &blocks,
+                         xo::FitMcvox{}))
+        return -1;
 
     if (nlut)
         XO_HIP(hipMemcpyAsync(ctx->lut, lut, (size_t)nlut * 4, hipMemcpyHostToDevice,
@@ -829,7 +964,7 @@ static int mcvox_run(xo_ctx *ctx, const xo_mcvox_cfg *cfg, const int32_t *voxels
     XO_HIP(hipMemsetAsync(ctx->counters, 0, sizeof(unsigned long long) * (1 + XO_STAT_COUNT),
                           ctx->stream));
     XO_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-    if (npackets > 0) XO_HIP(xo::launch_mcvox(P, blocks, ctx->stream));
+    if (npackets > 0) XO_HIP(xo::launch_mcvox(P, blocks, block, ctx->stream));
     XO_HIP(hipEventRecord(ctx->ev1, ctx->stream));
     unsigned long long stats[1 + XO_STAT_COUNT];
     XO_HIP(hipMemcpyAsync(accum, ctx->accum, naccum * 8, hipMemcpyDeviceToHost, ctx->stream));

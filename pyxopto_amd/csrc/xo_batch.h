@@ -30,7 +30,7 @@ struct BatchHdr {
     xo_detector top, bottom, specular;
     xo_source_fiber fiber;
     xo_fiber_axis fiber_axis;
-    xo_fluence fluence;         /* enabled 0: none */
+    FluenceL fluence;           /* enabled 0: none */
 };
 
 /* Host: instances of one class run the same branches of the transport
@@ -65,7 +65,7 @@ inline BatchHdr batch_header(const xo_batch_instance &I, const xo_detector det[3
     H.top.offset += accum_shift;
     H.bottom.offset += accum_shift;
     H.specular.offset += accum_shift;
-    H.fluence = I.fluence;
+    H.fluence = fluence_to_device(I.fluence);
     if (H.fluence.enabled != XO_FLUENCE_NONE) H.fluence.offset += accum_shift;
     return H;
 }

@@ -32,6 +32,7 @@ struct xo_ctx {
     hipStream_t stream = nullptr;
     uint32_t max_lanes = 0;
     uint32_t cus = 0;
+    uint32_t lds_per_cu = 65536;
     uint64_t *rng_x = nullptr;
     uint32_t *rng_a = nullptr;
     unsigned long long *counters = nullptr; /* [0] packet counter, [1..] stats */

@@ -13,6 +13,7 @@
 #include <stdint.h>
 
 #include "../../include/xomc.h"
+#include "xo_kernels.h"
 #include "xo_math.h"
 
 namespace xo {
@@ -292,48 +293,65 @@ XO_DEV void cache_flush(FluenceCache &c, unsigned long long *accum) {
 /* The weight a fluence accumulator adds for an absorbed weight w: w in
  * deposition mode, w / mua in fluence-rate mode (0 where mua is 0),
  * fluence.py:139-141. */
-template <class M = MathExact> XO_DEV float fluence_weight(const xo_fluence &F, float w, float mua) {
+template <class M = MathExact> XO_DEV float fluence_weight(const FluenceL &F, float w, float mua) {
     if (F.rate) w *= (mua != 0.0f) ? M::div(1.0f, mua) : 0.0f;
     return w;
 }
 
-/* Fluence deposit at a point: the Cartesian voxel of
- * mcsim_fluence_deposit_at (fluence.py:102-147) or the (r, z) cell of
- * fluencerz.py:112-160; mua is that of the medium the packet is in (used
- * in fluence-rate mode). Returns true if a non-zero integer was added. */
+/* Bin (x, y, z) of a point: the Cartesian voxel of mcsim_fluence_deposit_at
+ * (fluence.py:102-147) or the (r, 0, z) cell of fluencerz.py:112-160; false
+ * outside the grid. */
 template <class M = MathExact>
-XO_DEV bool fluence_deposit(const xo_fluence &F, unsigned long long *accum, float px,
-                            float py, float pz, float w, float mua,
-                            FluenceCache *cache = nullptr) {
-    uint64_t index;
+XO_DEV bool fluence_bin(const FluenceL &F, float px, float py, float pz, uint32_t &ix,
+                        uint32_t &iy, uint32_t &iz) {
+    const float ddx = px - F.top_left[0];
+    const float ddy = py - F.top_left[1];
+    const float ddz = pz - F.top_left[2];
+    const float fz = ddz * F.inv_step[2];
     if (F.enabled == XO_FLUENCE_XYZ) {
-        const float fx = (px - F.top_left[0]) * F.inv_step[0];
-        const float fy = (py - F.top_left[1]) * F.inv_step[1];
-        const float fz = (pz - F.top_left[2]) * F.inv_step[2];
-        if (!(fx >= 0.0f && fy >= 0.0f && fz >= 0.0f && fx < (float)F.shape[0] &&
-              fy < (float)F.shape[1] && fz < (float)F.shape[2]))
+        const float fx = ddx * F.inv_step[0];
+        const float fy = ddy * F.inv_step[1];
+        if (!(fx >= 0.0f && fy >= 0.0f && fz >= 0.0f && fx < F.shape[0] && fy < F.shape[1] &&
+              fz < F.shape[2]))
             return false;
-        const uint64_t ix = f2u_sat(fx), iy = f2u_sat(fy), iz = f2u_sat(fz);
-        index = (iz * F.shape[1] + iy) * F.shape[0] + ix;
-    } else if (F.enabled == XO_FLUENCE_RZ) {
-        const float ddx = px - F.top_left[0];
-        const float ddy = py - F.top_left[1];
-        const float r = M::sqrt(ddx * ddx + ddy * ddy);
-        const float ddz = pz - F.top_left[2];
-        const float fr = r * F.inv_step[0];
-        const float fz = ddz * F.inv_step[2];
-        if (!(fr >= 0.0f && fz >= 0.0f && fr < (float)F.shape[0] && fz < (float)F.shape[2]))
-            return false;
-        index = (uint64_t)f2u_sat(fz) * F.shape[0] + f2u_sat(fr);
-    } else {
-        return false;
+        ix = f2u_sat(fx);
+        iy = f2u_sat(fy);
+        iz = f2u_sat(fz);
+        return true;
     }
-    const uint32_t ui = f2u_sat(fluence_weight<M>(F, w, mua) * (float)F.k + 0.5f);
+    if (F.enabled == XO_FLUENCE_RZ) {
+        const float fr = M::sqrt(ddx * ddx + ddy * ddy) * F.inv_step[0];
+        if (!(fr >= 0.0f && fz >= 0.0f && fr < F.shape[0] && fz < F.shape[2])) return false;
+        ix = f2u_sat(fr);
+        iy = 0u;
+        iz = f2u_sat(fz);
+        return true;
+    }
+    return false;
+}
+
+/* Accumulator index of a fluence bin: x (or r) fastest. */
+XO_DEV uint64_t fluence_index(const FluenceL &F, uint32_t ix, uint32_t iy, uint32_t iz) {
+    return F.offset + ((uint64_t)iz * F.ny + iy) * F.nx + ix;
+}
+
+/* Integer weight of a deposit; mua is that of the medium the packet is in
+ * (used in fluence-rate mode). */
+template <class M = MathExact>
+XO_DEV uint32_t fluence_integer(const FluenceL &F, float w, float mua) {
+    return f2u_sat(fluence_weight<M>(F, w, mua) * F.k + 0.5f);
+}
+
+/* Fluence deposit at a point. Returns true if a non-zero integer was
+ * added. */
+template <class M = MathExact>
+XO_DEV bool fluence_deposit(const FluenceL &F, unsigned long long *accum, float px,
+                            float py, float pz, float w, float mua) {
+    uint32_t ix, iy, iz;
+    if (!fluence_bin<M>(F, px, py, pz, ix, iy, iz)) return false;
+    const uint32_t ui = fluence_integer<M>(F, w, mua);
     if (ui == 0u) return false;
-    if (cache)
-        cache_add(*cache, accum, F.offset + index, ui);
-    else
-        atomicAdd(&accum[F.offset + index], (unsigned long long)ui);
+    atomicAdd(&accum[fluence_index(F, ix, iy, iz)], (unsigned long long)ui);
     return true;
 }
 
@@ -353,7 +371,7 @@ template <class T> XO_DEV const T &lds_fresh(const T &ref) {
  * LDS once per block. */
 struct LayerEventCfgL {
     xo_detector top, bottom, specular;
-    xo_fluence fluence;
+    FluenceL fluence;
     xo_source_line line;
     xo_source_fiber fiber;
     xo_fiber_axis fiber_axis;
@@ -361,37 +379,51 @@ struct LayerEventCfgL {
 
 struct VoxEventCfgL {
     xo_detector top, bottom, specular;
-    xo_fluence fluence;
+    FluenceL fluence;
     xo_source_line line;
     xo_source_gaussian gaussian;
 };
 
-/* fluence_deposit for a Cartesian grid whose bins in the box
- * [box, box + (bx, by, bz)) are held in LDS (sbox, x fastest): the same
- * index and integer as fluence_deposit, added to the box when the bin lies
- * in it, to accum through the lane's cache otherwise. */
+/* fluence_deposit of the single-simulation kernels: the same bin and
+ * integer, added in LDS (wbins) when the bin lies in the block's window, to
+ * accum through the lane's cache otherwise. A beam's first interactions
+ * land in a handful of bins, and the device adds at most 2.4e10 u64 per
+ * second to memory, 8.5e8 if 64 bins take them all, against 2.6e12 in LDS
+ * (3e11 into a single bin). */
 template <class M = MathExact>
-XO_DEV bool fluence_deposit_boxed(const xo_fluence &F, unsigned long long *accum,
-                                  unsigned long long *sbox, const int32_t box[3], int32_t bx,
-                                  int32_t by, int32_t bz, float px, float py, float pz,
-                                  float w, float mua, FluenceCache &cache) {
-    const float fx = (px - F.top_left[0]) * F.inv_step[0];
-    const float fy = (py - F.top_left[1]) * F.inv_step[1];
-    const float fz = (pz - F.top_left[2]) * F.inv_step[2];
-    if (!(fx >= 0.0f && fy >= 0.0f && fz >= 0.0f && fx < (float)F.shape[0] &&
-          fy < (float)F.shape[1] && fz < (float)F.shape[2]))
-        return false;
-    const uint32_t ix = f2u_sat(fx), iy = f2u_sat(fy), iz = f2u_sat(fz);
-    const uint32_t ui = f2u_sat(fluence_weight<M>(F, w, mua) * (float)F.k + 0.5f);
+XO_DEV bool fluence_deposit_win(const FluenceL &F, unsigned long long *accum,
+                                unsigned long long *wbins, float px, float py, float pz, float w,
+                                float mua, FluenceCache &cache) {
+    uint32_t ix, iy, iz;
+    if (!fluence_bin<M>(F, px, py, pz, ix, iy, iz)) return false;
+    const uint32_t ui = fluence_integer<M>(F, w, mua);
     if (ui == 0u) return false;
-    const uint32_t rx = ix - (uint32_t)box[0], ry = iy - (uint32_t)box[1],
-                   rz = iz - (uint32_t)box[2];
-    if (rx < (uint32_t)bx && ry < (uint32_t)by && rz < (uint32_t)bz)
-        atomicAdd(&sbox[(rz * (uint32_t)by + ry) * (uint32_t)bx + rx], (unsigned long long)ui);
-    else
-        cache_add(cache, accum, F.offset + ((uint64_t)iz * F.shape[1] + iy) * F.shape[0] + ix,
-                  ui);
+    if (wbins) {
+        const uint32_t rx = ix - F.origin[0], ry = iy - F.origin[1], rz = iz - F.origin[2];
+        if (rx < F.ext[0] && ry < F.ext[1] && rz < F.ext[2]) {
+            atomicAdd(&wbins[(rz * F.ext[1] + ry) * F.ext[0] + rx], (unsigned long long)ui);
+            return true;
+        }
+    }
+    cache_add(cache, accum, fluence_index(F, ix, iy, iz), ui);
     return true;
+}
+
+/* The block's window added to accum; blocks start at different bins, so
+ * that those ending together do not queue at the same one. */
+XO_DEV void fluence_window_flush(const FluenceL &F, unsigned long long *accum,
+                                 const unsigned long long *wbins) {
+    const uint32_t first = (uint32_t)(((uint64_t)blockIdx.x * F.bins) / gridDim.x);
+    for (uint32_t k = threadIdx.x; k < F.bins; k += blockDim.x) {
+        const uint32_t i = first + k < F.bins ? first + k : first + k - F.bins;
+        const unsigned long long v = wbins[i];
+        if (!v) continue;
+        const uint32_t row = i / F.ext[0];
+        atomicAdd(&accum[fluence_index(F, F.origin[0] + i % F.ext[0],
+                                       F.origin[1] + row % F.ext[1],
+                                       F.origin[2] + row / F.ext[1])],
+                  v);
+    }
 }
 
 /* Phase-function parameters of one layer/material, read from LDS. */

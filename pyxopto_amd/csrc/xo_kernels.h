@@ -12,6 +12,7 @@
 
 /* Threads per block: 4 wave64 wavefronts. */
 #define XO_BLOCK 256
+#define XO_MAX_BLOCK 1024 /* of a run with a fluence window in LDS */
 
 /* Per-run counters accumulated by the kernels. */
 enum {
@@ -32,6 +33,41 @@ enum {
 
 namespace xo {
 
+/* A fluence grid as the kernels read it per deposit, in five 16-byte words.
+ * origin, ext, bins: the box of bins (x or r, y, z; x fastest) that a block
+ * of a single-simulation kernel accumulates in LDS and adds to the
+ * accumulator once; bins 0: none. */
+struct alignas(16) FluenceL {
+    float top_left[3];
+    float k;               /* float to integer weight                     */
+    float inv_step[3];
+    int32_t enabled;       /* enum xo_fluence_kind                        */
+    float shape[3];
+    uint32_t offset;
+    uint32_t origin[3];
+    uint32_t nx;           /* bins of a row ...                           */
+    uint32_t ext[3];
+    uint32_t ny;           /* ... and rows of a slice (1 for r-z)         */
+    uint32_t bins;
+    int32_t rate;
+};
+
+inline FluenceL fluence_to_device(const xo_fluence &F) {
+    FluenceL o = {};
+    for (int k = 0; k < 3; ++k) {
+        o.top_left[k] = F.top_left[k];
+        o.inv_step[k] = F.inv_step[k];
+        o.shape[k] = (float)F.shape[k];
+    }
+    o.k = (float)F.k;
+    o.enabled = F.enabled;
+    o.offset = F.offset;
+    o.nx = F.shape[0];
+    o.ny = F.enabled == XO_FLUENCE_XYZ ? F.shape[1] : 1u;
+    o.rate = F.rate;
+    return o;
+}
+
 struct McmlParams {
     xo_mcml_cfg cfg;
     xo_trace trace;        /* max_events 0: no trace                      */
@@ -49,6 +85,7 @@ struct McmlParams {
     uint32_t flags;
     uint32_t lds_bins;
     uint32_t lds_lut;
+    FluenceL fluence;      /* the grid of cfg.fluence, with its window    */
 };
 
 struct McvoxParams {
@@ -69,24 +106,23 @@ struct McvoxParams {
     uint32_t flags;
     uint32_t lds_bins;
     uint32_t lds_lut;
-    /* Cartesian fluence bins of one kFlBox-sized box of the grid (origin
-     * fl_box, in bins) accumulate in LDS and are added to accum once per
-     * block: the box around the beam's entry takes a large share of the
-     * deposits. fl_box_on 0: every deposit goes to accum. */
-    int32_t fl_box[3];
-    uint32_t fl_box_on;
+    FluenceL fluence;      /* the grid of cfg.fluence, with its window    */
 };
 
-/* Extent of the LDS fluence box (x, y, z bins). */
-constexpr int32_t kFlBoxX = 16, kFlBoxY = 16, kFlBoxZ = 8;
-constexpr uint32_t kFlBoxBins = kFlBoxX * kFlBoxY * kFlBoxZ;
+/* Largest window: zeroing and adding it up costs every block about a
+ * microsecond per 4096 bins. */
+constexpr uint32_t kFluenceWindowMax = 10240;
 
 size_t mcml_lds_bytes(const McmlParams &P);
 size_t mcvox_lds_bytes(const McvoxParams &P);
-hipError_t launch_mcml(const McmlParams &P, uint32_t blocks, hipStream_t stream);
-hipError_t launch_mcvox(const McvoxParams &P, uint32_t blocks, hipStream_t stream);
-hipError_t occupancy_mcml(int pf_kind, size_t lds, bool fast, int *blocks_per_cu);
-hipError_t occupancy_mcvox(int pf_kind, size_t lds, bool fast, int *blocks_per_cu);
+/* Blocks of `block` threads (at most XO_MAX_BLOCK). */
+hipError_t launch_mcml(const McmlParams &P, uint32_t blocks, uint32_t block, hipStream_t stream);
+hipError_t launch_mcvox(const McvoxParams &P, uint32_t blocks, uint32_t block,
+                        hipStream_t stream);
+/* Resident blocks per CU of the build that launch_mcml / launch_mcvox would
+ * run for P, at this block size and P's LDS. */
+hipError_t occupancy_mcml(const McmlParams &P, uint32_t block, int *blocks_per_cu);
+hipError_t occupancy_mcvox(const McvoxParams &P, uint32_t block, int *blocks_per_cu);
 
 } // namespace xo
 

@@ -46,14 +46,17 @@ constexpr uint32_t kDeferMin = 12, kDeferWait = 8;
 /* Transport rounds (B then C) per loop iteration of the layered kernel. */
 constexpr int kRoundsPerIteration = 6;
 
-template <int PF, int METHOD, bool TRACE, class M>
-__global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
+/* FLU: built with the fluence deposit. Without it the loop keeps to 64-72
+ * registers (7 waves per SIMD); traced runs have one build for both. */
+template <int PF, int METHOD, bool TRACE, bool FLU, class M>
+__global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ BlockStats sstats;
     __shared__ LayerEventCfgL sev;
     LayerL *sl = reinterpret_cast<LayerL *>(smem);
-    unsigned long long *sbins =
+    unsigned long long *swin =
         reinterpret_cast<unsigned long long *>(smem + XO_MAX_LAYERS * sizeof(LayerL));
+    unsigned long long *sbins = swin + P.fluence.bins;
     float *slut = reinterpret_cast<float *>(sbins + P.lds_bins);
 
     const uint32_t tid = threadIdx.x;
@@ -79,14 +82,14 @@ __global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
         o.mus = L.mus;
         sl[tid] = o;
     }
-    for (uint32_t i = tid; i < P.lds_bins; i += XO_BLOCK) sbins[i] = 0ull;
-    for (uint32_t i = tid; i < P.lds_lut; i += XO_BLOCK) slut[i] = P.lut[i];
+    for (uint32_t i = tid; i < P.fluence.bins + P.lds_bins; i += blockDim.x) swin[i] = 0ull;
+    for (uint32_t i = tid; i < P.lds_lut; i += blockDim.x) slut[i] = P.lut[i];
     if (tid < XO_STAT_COUNT) sstats.v[tid] = 0ull;
     if (tid == 0) {
         sev.top = P.cfg.top;
         sev.bottom = P.cfg.bottom;
         sev.specular = P.cfg.specular;
-        sev.fluence = P.cfg.fluence;
+        sev.fluence = P.fluence;
         sev.line = P.cfg.source;
         sev.fiber = P.cfg.fiber;
         sev.fiber_axis = P.cfg.fiber_axis;
@@ -96,7 +99,7 @@ __global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
     const Bins bins{P.lds_bins ? sbins : nullptr, P.accum};
     const float *lut = P.lds_lut ? slut : P.lut;
 
-    const uint32_t gid = blockIdx.x * XO_BLOCK + tid;
+    const uint32_t gid = blockIdx.x * blockDim.x + tid;
     const bool lane_ok = gid < P.lanes;
     const bool static_sched = (P.flags & XO_FLAG_STATIC_SCHEDULE) != 0u;
     const bool keyed = (P.flags & XO_FLAG_PACKET_KEYED) != 0u;
@@ -121,8 +124,14 @@ __global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
     const float spz = sp[2];
     const float w_min = P.cfg.w_min, chance = P.cfg.lottery_chance;
     const int use_lottery = P.cfg.use_lottery;
-    const bool use_fluence = P.cfg.fluence.enabled != XO_FLUENCE_NONE;
+    const bool use_fluence = FLU && P.cfg.fluence.enabled != XO_FLUENCE_NONE;
     const bool use_specular = P.cfg.specular.kind != XO_DET_NONE;
+    FluenceCache fcache;
+    unsigned long long *wbins = P.fluence.bins ? swin : nullptr;
+    auto deposit_fluence = [&](float qx, float qy, float qz, float wgt, float mua) {
+        return fluence_deposit_win<M>(lds_fresh(sev.fluence), P.accum, wbins, qx, qy, qz, wgt,
+                                      mua, fcache);
+    };
 
     bool active = lane_ok;
     WaveDispenser wq;
@@ -255,8 +264,7 @@ __global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
                     (mua != 0.0f)
                         ? step - M::div(-M::log_unit(1.0f - rng_next(x, a) * fraction), mua)
                         : 0.0f;
-                if (fluence_deposit<M>(lds_fresh(sev.fluence), P.accum, px - back * dx,
-                                       py - back * dy, pz - back * dz, deposit, mua))
+                if (deposit_fluence(px - back * dx, py - back * dy, pz - back * dz, deposit, mua))
                     st[XO_STAT_DEPOSITS]++;
             }
         };
@@ -376,9 +384,7 @@ __global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
                     const float deposit = w;
                     w -= deposit;
                     if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
-                    if (use_fluence &&
-                        fluence_deposit<M>(lds_fresh(sev.fluence), P.accum, px, py, pz, deposit,
-                                           L.mua))
+                    if (use_fluence && deposit_fluence(px, py, pz, deposit, L.mua))
                         st[XO_STAT_DEPOSITS]++;
                     done = true;
                 } else {
@@ -386,9 +392,7 @@ __global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
                         const float deposit = w * lt.w;
                         w -= deposit;
                         if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
-                        if (use_fluence &&
-                            fluence_deposit<M>(lds_fresh(sev.fluence), P.accum, px, py, pz, deposit,
-                                               L.mua))
+                        if (use_fluence && deposit_fluence(px, py, pz, deposit, L.mua))
                             st[XO_STAT_DEPOSITS]++;
                     }
                     float xi_fi;
@@ -403,15 +407,17 @@ __global__ void __launch_bounds__(XO_BLOCK) mcml_kernel(const McmlParams P) {
         }
     }
 
+    if (FLU) cache_flush(fcache, P.accum);
     if (lane_ok) {
         if (!keyed) P.rng_x[gid] = x;
         if (st[XO_STAT_PACKETS]) st[XO_STAT_THREADS] = 1;
     }
     stats_flush(&sstats, st, P.stats);
     if (P.lds_bins) {
-        for (uint32_t i = tid; i < P.lds_bins; i += XO_BLOCK)
+        for (uint32_t i = tid; i < P.lds_bins; i += blockDim.x)
             if (sbins[i]) atomicAdd(&P.accum[i], sbins[i]);
     }
+    if (FLU) fluence_window_flush(P.fluence, P.accum, swin);
 }
 
 /* ------------------------------------------------------------------ */
@@ -480,14 +486,14 @@ constexpr uint32_t kVoxDeferMin = 24, kVoxDeferWait = 8;
 constexpr int kVoxRoundsPerIteration = 4;
 
 template <int PF, int METHOD, bool TRACE, class M>
-__global__ void __launch_bounds__(XO_BLOCK) mcvox_kernel(const McvoxParams P) {
+__global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ BlockStats sstats;
     __shared__ VoxEventCfgL sev;
     MaterialL *sm = reinterpret_cast<MaterialL *>(smem);
-    unsigned long long *sfl = reinterpret_cast<unsigned long long *>(
+    unsigned long long *swin = reinterpret_cast<unsigned long long *>(
         smem + XO_MAX_MATERIALS * sizeof(MaterialL));
-    unsigned long long *sbins = sfl + (P.fl_box_on ? kFlBoxBins : 0u);
+    unsigned long long *sbins = swin + P.fluence.bins;
     float *slut = reinterpret_cast<float *>(sbins + P.lds_bins);
 
     const uint32_t tid = threadIdx.x;
@@ -509,16 +515,14 @@ __global__ void __launch_bounds__(XO_BLOCK) mcvox_kernel(const McvoxParams P) {
         o.mus = Mi.mus;
         sm[tid] = o;
     }
-    for (uint32_t i = tid; i < P.lds_bins; i += XO_BLOCK) sbins[i] = 0ull;
-    if (P.fl_box_on)
-        for (uint32_t i = tid; i < kFlBoxBins; i += XO_BLOCK) sfl[i] = 0ull;
-    for (uint32_t i = tid; i < P.lds_lut; i += XO_BLOCK) slut[i] = P.lut[i];
+    for (uint32_t i = tid; i < P.fluence.bins + P.lds_bins; i += blockDim.x) swin[i] = 0ull;
+    for (uint32_t i = tid; i < P.lds_lut; i += blockDim.x) slut[i] = P.lut[i];
     if (tid < XO_STAT_COUNT) sstats.v[tid] = 0ull;
     if (tid == 0) {
         sev.top = P.cfg.top;
         sev.bottom = P.cfg.bottom;
         sev.specular = P.cfg.specular;
-        sev.fluence = P.cfg.fluence;
+        sev.fluence = P.fluence;
         sev.line = P.cfg.line;
         sev.gaussian = P.cfg.gaussian;
     }
@@ -536,18 +540,14 @@ __global__ void __launch_bounds__(XO_BLOCK) mcvox_kernel(const McvoxParams P) {
         g.shape[k] = P.cfg.voxels.shape[k];
     }
     const bool use_fluence = P.cfg.fluence.enabled != 0;
-    /* a fluence deposit: through the LDS box when there is one */
     FluenceCache fcache;
+    unsigned long long *wbins = P.fluence.bins ? swin : nullptr;
     auto deposit_fluence = [&](float qx, float qy, float qz, float wgt, float mua) {
-        if (P.fl_box_on)
-            return fluence_deposit_boxed<M>(lds_fresh(sev.fluence), P.accum, sfl, P.fl_box,
-                                            kFlBoxX, kFlBoxY, kFlBoxZ, qx, qy, qz, wgt, mua,
-                                            fcache);
-        return fluence_deposit<M>(lds_fresh(sev.fluence), P.accum, qx, qy, qz, wgt, mua,
-                                  &fcache);
+        return fluence_deposit_win<M>(lds_fresh(sev.fluence), P.accum, wbins, qx, qy, qz, wgt,
+                                      mua, fcache);
     };
 
-    const uint32_t gid = blockIdx.x * XO_BLOCK + tid;
+    const uint32_t gid = blockIdx.x * blockDim.x + tid;
     const bool lane_ok = gid < P.lanes;
     const bool static_sched = (P.flags & XO_FLAG_STATIC_SCHEDULE) != 0u;
     const bool keyed = (P.flags & XO_FLAG_PACKET_KEYED) != 0u;
@@ -922,167 +922,98 @@ __global__ void __launch_bounds__(XO_BLOCK) mcvox_kernel(const McvoxParams P) {
     }
     stats_flush(&sstats, st, P.stats);
     if (P.lds_bins) {
-        for (uint32_t i = tid; i < P.lds_bins; i += XO_BLOCK)
+        for (uint32_t i = tid; i < P.lds_bins; i += blockDim.x)
             if (sbins[i]) atomicAdd(&P.accum[i], sbins[i]);
     }
-    if (P.fl_box_on) {
-        const xo_fluence &F = P.cfg.fluence;
-        for (uint32_t i = tid; i < kFlBoxBins; i += XO_BLOCK) {
-            if (!sfl[i]) continue;
-            const uint64_t ix = (uint64_t)P.fl_box[0] + i % kFlBoxX;
-            const uint64_t iy = (uint64_t)P.fl_box[1] + (i / kFlBoxX) % kFlBoxY;
-            const uint64_t iz = (uint64_t)P.fl_box[2] + i / (kFlBoxX * kFlBoxY);
-            atomicAdd(&P.accum[F.offset + (iz * F.shape[1] + iy) * F.shape[0] + ix], sfl[i]);
-        }
-    }
+    fluence_window_flush(P.fluence, P.accum, swin);
 }
 
 /* ------------------------------------------------------------------ */
 /* launchers                                                          */
 /* ------------------------------------------------------------------ */
 size_t mcml_lds_bytes(const McmlParams &P) {
-    return XO_MAX_LAYERS * sizeof(LayerL) + 8u * P.lds_bins + 4u * P.lds_lut;
+    return XO_MAX_LAYERS * sizeof(LayerL) + 8u * (P.fluence.bins + P.lds_bins) + 4u * P.lds_lut;
 }
 
 size_t mcvox_lds_bytes(const McvoxParams &P) {
-    return XO_MAX_MATERIALS * sizeof(MaterialL) + (P.fl_box_on ? 8u * kFlBoxBins : 0u) +
-           8u * P.lds_bins + 4u * P.lds_lut;
+    return XO_MAX_MATERIALS * sizeof(MaterialL) + 8u * (P.fluence.bins + P.lds_bins) +
+           4u * P.lds_lut;
 }
 
-template <int PF, bool TRACE, class M>
-static hipError_t launch_mcml_pf(const McmlParams &P, uint32_t blocks, size_t lds,
-                                 hipStream_t stream) {
+/* The build of a kernel for a run's phase function, stepping method and
+ * arithmetic (traced runs use the exact arithmetic whatever the flags say);
+ * null for an unknown one. */
+template <int PF, int METHOD, class Params> struct KernelOf;
+template <int PF, int METHOD> struct KernelOf<PF, METHOD, McmlParams> {
+    template <bool TRACE, class M> static const void *get(const McmlParams &P) {
+        if (TRACE || P.cfg.fluence.enabled != XO_FLUENCE_NONE)
+            return reinterpret_cast<const void *>(&mcml_kernel<PF, METHOD, TRACE, true, M>);
+        return reinterpret_cast<const void *>(&mcml_kernel<PF, METHOD, TRACE, TRACE, M>);
+    }
+};
+template <int PF, int METHOD> struct KernelOf<PF, METHOD, McvoxParams> {
+    template <bool TRACE, class M> static const void *get(const McvoxParams &) {
+        return reinterpret_cast<const void *>(&mcvox_kernel<PF, METHOD, TRACE, M>);
+    }
+};
+
+template <int PF, int METHOD, class Params> static const void *kernel_arith(const Params &P) {
+    using K = KernelOf<PF, METHOD, Params>;
+    if (P.trace.max_events > 0) return K::template get<true, MathExact>(P);
+    if (P.flags & XO_FLAG_FAST_MATH) return K::template get<false, MathFast>(P);
+    return K::template get<false, MathExact>(P);
+}
+
+template <int PF, class Params> static const void *kernel_method(const Params &P) {
     switch (P.cfg.method) {
-    case XO_METHOD_AW:
-        hipLaunchKernelGGL((mcml_kernel<PF, XO_METHOD_AW, TRACE, M>), dim3(blocks),
-                           dim3(XO_BLOCK), lds, stream, P);
-        break;
-    case XO_METHOD_AR:
-        hipLaunchKernelGGL((mcml_kernel<PF, XO_METHOD_AR, TRACE, M>), dim3(blocks),
-                           dim3(XO_BLOCK), lds, stream, P);
-        break;
-    case XO_METHOD_MBL:
-        hipLaunchKernelGGL((mcml_kernel<PF, XO_METHOD_MBL, TRACE, M>), dim3(blocks),
-                           dim3(XO_BLOCK), lds, stream, P);
-        break;
-    default:
-        return hipErrorInvalidValue;
+    case XO_METHOD_AW: return kernel_arith<PF, XO_METHOD_AW>(P);
+    case XO_METHOD_AR: return kernel_arith<PF, XO_METHOD_AR>(P);
+    case XO_METHOD_MBL: return kernel_arith<PF, XO_METHOD_MBL>(P);
+    default: return nullptr;
     }
-    return hipGetLastError();
 }
 
-/* Traced runs use the exact arithmetic whatever the flags say. */
-template <int PF>
-static hipError_t launch_mcml_pf(const McmlParams &P, uint32_t blocks, size_t lds,
-                                 hipStream_t stream) {
-    if (P.trace.max_events > 0)
-        return launch_mcml_pf<PF, true, MathExact>(P, blocks, lds, stream);
-    if (P.flags & XO_FLAG_FAST_MATH)
-        return launch_mcml_pf<PF, false, MathFast>(P, blocks, lds, stream);
-    return launch_mcml_pf<PF, false, MathExact>(P, blocks, lds, stream);
-}
-
-hipError_t launch_mcml(const McmlParams &P, uint32_t blocks, hipStream_t stream) {
-    size_t lds = mcml_lds_bytes(P);
+template <class Params> static const void *kernel_for(const Params &P) {
     switch (P.cfg.pf_kind) {
-    case XO_PF_HG:
-        return launch_mcml_pf<XO_PF_HG>(P, blocks, lds, stream);
-    case XO_PF_MHG:
-        return launch_mcml_pf<XO_PF_MHG>(P, blocks, lds, stream);
-    case XO_PF_LUT:
-        return launch_mcml_pf<XO_PF_LUT>(P, blocks, lds, stream);
-    default:
-        return hipErrorInvalidValue;
+    case XO_PF_HG: return kernel_method<XO_PF_HG>(P);
+    case XO_PF_MHG: return kernel_method<XO_PF_MHG>(P);
+    case XO_PF_LUT: return kernel_method<XO_PF_LUT>(P);
+    default: return nullptr;
     }
 }
 
-template <int PF, bool TRACE, class M>
-static hipError_t launch_mcvox_pf(const McvoxParams &P, uint32_t blocks, size_t lds,
-                                 hipStream_t stream) {
-    switch (P.cfg.method) {
-    case XO_METHOD_AW:
-        hipLaunchKernelGGL((mcvox_kernel<PF, XO_METHOD_AW, TRACE, M>), dim3(blocks),
-                           dim3(XO_BLOCK), lds, stream, P);
-        break;
-    case XO_METHOD_AR:
-        hipLaunchKernelGGL((mcvox_kernel<PF, XO_METHOD_AR, TRACE, M>), dim3(blocks),
-                           dim3(XO_BLOCK), lds, stream, P);
-        break;
-    case XO_METHOD_MBL:
-        hipLaunchKernelGGL((mcvox_kernel<PF, XO_METHOD_MBL, TRACE, M>), dim3(blocks),
-                           dim3(XO_BLOCK), lds, stream, P);
-        break;
-    default:
-        return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+template <class Params>
+static hipError_t launch(const Params &P, size_t lds, uint32_t blocks, uint32_t block,
+                         hipStream_t stream) {
+    const void *fn = kernel_for(P);
+    if (!fn || block > XO_MAX_BLOCK) return hipErrorInvalidValue;
+    void *args[] = {const_cast<Params *>(&P)};
+    return hipLaunchKernel(fn, dim3(blocks), dim3(block), args, lds, stream);
 }
 
-/* Traced runs use the exact arithmetic whatever the flags say. */
-template <int PF>
-static hipError_t launch_mcvox_pf(const McvoxParams &P, uint32_t blocks, size_t lds,
-                                 hipStream_t stream) {
-    if (P.trace.max_events > 0)
-        return launch_mcvox_pf<PF, true, MathExact>(P, blocks, lds, stream);
-    if (P.flags & XO_FLAG_FAST_MATH)
-        return launch_mcvox_pf<PF, false, MathFast>(P, blocks, lds, stream);
-    return launch_mcvox_pf<PF, false, MathExact>(P, blocks, lds, stream);
+template <class Params>
+static hipError_t occupancy(const Params &P, size_t lds, uint32_t block, int *blocks_per_cu) {
+    const void *fn = kernel_for(P);
+    if (!fn || block > XO_MAX_BLOCK) return hipErrorInvalidValue;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, (int)block, lds);
 }
 
-hipError_t launch_mcvox(const McvoxParams &P, uint32_t blocks, hipStream_t stream) {
-    size_t lds = mcvox_lds_bytes(P);
-    switch (P.cfg.pf_kind) {
-    case XO_PF_HG:
-        return launch_mcvox_pf<XO_PF_HG>(P, blocks, lds, stream);
-    case XO_PF_MHG:
-        return launch_mcvox_pf<XO_PF_MHG>(P, blocks, lds, stream);
-    case XO_PF_LUT:
-        return launch_mcvox_pf<XO_PF_LUT>(P, blocks, lds, stream);
-    default:
-        return hipErrorInvalidValue;
-    }
+hipError_t launch_mcml(const McmlParams &P, uint32_t blocks, uint32_t block,
+                       hipStream_t stream) {
+    return launch(P, mcml_lds_bytes(P), blocks, block, stream);
 }
 
-/* Blocks per CU of the albedo-weight build of the arithmetic that will
- * run (it stands for all three methods: same registers within a few). */
-template <class M>
-static hipError_t occupancy_mcml_m(int pf_kind, size_t lds, int *blocks_per_cu) {
-    switch (pf_kind) {
-    case XO_PF_MHG:
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, mcml_kernel<XO_PF_MHG, XO_METHOD_AW, false, M>, XO_BLOCK, lds);
-    case XO_PF_LUT:
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, mcml_kernel<XO_PF_LUT, XO_METHOD_AW, false, M>, XO_BLOCK, lds);
-    default:
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, mcml_kernel<XO_PF_HG, XO_METHOD_AW, false, M>, XO_BLOCK, lds);
-    }
+hipError_t launch_mcvox(const McvoxParams &P, uint32_t blocks, uint32_t block,
+                        hipStream_t stream) {
+    return launch(P, mcvox_lds_bytes(P), blocks, block, stream);
 }
 
-template <class M>
-static hipError_t occupancy_mcvox_m(int pf_kind, size_t lds, int *blocks_per_cu) {
-    switch (pf_kind) {
-    case XO_PF_MHG:
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, mcvox_kernel<XO_PF_MHG, XO_METHOD_AW, false, M>, XO_BLOCK, lds);
-    case XO_PF_LUT:
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, mcvox_kernel<XO_PF_LUT, XO_METHOD_AW, false, M>, XO_BLOCK, lds);
-    default:
-        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            blocks_per_cu, mcvox_kernel<XO_PF_HG, XO_METHOD_AW, false, M>, XO_BLOCK, lds);
-    }
+hipError_t occupancy_mcml(const McmlParams &P, uint32_t block, int *blocks_per_cu) {
+    return occupancy(P, mcml_lds_bytes(P), block, blocks_per_cu);
 }
 
-hipError_t occupancy_mcml(int pf_kind, size_t lds, bool fast, int *blocks_per_cu) {
-    return fast ? occupancy_mcml_m<MathFast>(pf_kind, lds, blocks_per_cu)
-                : occupancy_mcml_m<MathExact>(pf_kind, lds, blocks_per_cu);
-}
-
-hipError_t occupancy_mcvox(int pf_kind, size_t lds, bool fast, int *blocks_per_cu) {
-    return fast ? occupancy_mcvox_m<MathFast>(pf_kind, lds, blocks_per_cu)
-                : occupancy_mcvox_m<MathExact>(pf_kind, lds, blocks_per_cu);
+hipError_t occupancy_mcvox(const McvoxParams &P, uint32_t block, int *blocks_per_cu) {
+    return occupancy(P, mcvox_lds_bytes(P), block, blocks_per_cu);
 }
 
 } // namespace xo

@@ -302,6 +302,7 @@ int launch_vox(xo_server *S, Request &R, uint64_t first, uint64_t count,
     P.cfg = R.vcfg;
     P.cfg.packet_seed = R.vcfg.packet_seed;
     P.cfg.first_packet = first;
+    P.fluence = xo::fluence_to_device(R.vcfg.fluence);
     P.table = S->ctx->table;
     P.voxels = S->vox + R.vox_off;
     P.lut = R.lut_n ? S->lut + R.lut_off : nullptr;
@@ -315,14 +316,13 @@ int launch_vox(xo_server *S, Request &R, uint64_t first, uint64_t count,
     P.lds_bins = R.lds_bins;
     P.lds_lut = (R.lut_n && R.lut_n <= XO_LDS_LUT_MAX) ? (uint32_t)R.lut_n : 0u;
     int bpc = 1;
-    XO_CHECK(xo::occupancy_mcvox(R.vcfg.pf_kind, xo::mcvox_lds_bytes(P),
-                                 S->opts.fast_math != 0, &bpc));
+    XO_CHECK(xo::occupancy_mcvox(P, XO_BLOCK, &bpc));
     uint64_t resident = (uint64_t)std::max(bpc, 1) * S->ctx->cus * XO_BLOCK;
     uint64_t lanes = std::min<uint64_t>(std::min<uint64_t>(count, resident), S->opts.vox_lanes);
     lanes = std::max<uint64_t>(lanes, 64u);
     P.lanes = (uint32_t)lanes;
     XO_CHECK(xo::launch_zero_u32((uint32_t *)counters, 2 * kCounterWords, stream));
-    XO_CHECK(xo::launch_mcvox(P, (uint32_t)((lanes + XO_BLOCK - 1) / XO_BLOCK), stream));
+    XO_CHECK(xo::launch_mcvox(P, (uint32_t)((lanes + XO_BLOCK - 1) / XO_BLOCK), XO_BLOCK, stream));
     return 0;
 }
 
