@@ -277,7 +277,7 @@ batch_kernel(const BatchParams P) {
             /* the wait count of the first active lane (lanes that were idle
              * hold stale counts), so the decision is wave-uniform */
             const uint32_t bw = (uint32_t)__builtin_amdgcn_readfirstlane((int)bwait);
-            const bool run_b = nb != 0 && (nb >= P.defer_min || nb == nal || bw >= kDeferWait);
+            const bool run_b = nb != 0 && (64u * nb >= P.defer_min * nal || nb == nal || bw >= kDeferWait);
             bwait = (nb != 0 && !run_b) ? bw + 1u : 0u;
             if (run_b && pend == kEvBoundary) {
                 /* (A) the step as drawn, clipped to the boundary it reaches */

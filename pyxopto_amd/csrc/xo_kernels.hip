@@ -298,7 +298,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
             const uint32_t nb = (uint32_t)__builtin_popcountll(__ballot(pend == kEvBoundary));
             const uint32_t nal = (uint32_t)__builtin_popcountll(__ballot(true));
             const uint32_t bw = (uint32_t)__builtin_amdgcn_readfirstlane((int)bwait);
-            const bool run_b = nb != 0 && (nb >= kDeferMin || nb == nal || bw >= kDeferWait);
+            const bool run_b = nb != 0 && (64u * nb >= kDeferMin * nal || bw >= kDeferWait);
             bwait = (nb != 0 && !run_b) ? bw + 1u : 0u;
             if (run_b && pend == kEvBoundary) {
                 /* (A) the step as drawn, clipped to the boundary it reaches */
@@ -723,8 +723,8 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
          * wave, so the wait count stays wave-uniform. ---- */
         const uint32_t n_int = (uint32_t)__builtin_popcountll(__ballot(alive && pend_int));
         const uint32_t n_alive = (uint32_t)__builtin_popcountll(__ballot(alive));
-        const bool run_int = n_int != 0 && (n_int >= kVoxDeferMin || n_int == n_alive ||
-                                            iwait >= kVoxDeferWait);
+        const bool run_int =
+            n_int != 0 && (64u * n_int >= kVoxDeferMin * n_alive || iwait >= kVoxDeferWait);
         iwait = (n_int != 0 && !run_int) ? iwait + 1u : 0u;
         if (!alive) continue;
 
