@@ -29,74 +29,78 @@ struct BatchBlockStats {
     unsigned long long v[XO_STAT_COUNT];
 };
 
-/* Phase-function sampling by the instance's kind. */
+/* Phase-function sampling by the lane's instance's kind. */
 template <class M>
 XO_DEV float pf_sample_rt(int kind, const PfL &pf, const float *lut, uint64_t &x, uint32_t a,
                           float &xi_fi) {
-    if (kind == XO_PF_HG) return pf_sample<XO_PF_HG, M>(pf, lut, x, a, xi_fi);
-    if (kind == XO_PF_MHG) return pf_sample<XO_PF_MHG, M>(pf, lut, x, a, xi_fi);
-    return pf_sample<XO_PF_LUT, M>(pf, lut, x, a, xi_fi);
+    if (kind == XO_PF_HG) return pf_sample<XO_PF_HG, true, M>(pf, lut, x, a, xi_fi);
+    if (kind == XO_PF_MHG) return pf_sample<XO_PF_MHG, true, M>(pf, lut, x, a, xi_fi);
+    return pf_sample<XO_PF_LUT, true, M>(pf, lut, x, a, xi_fi);
 }
+
+/* What the rounds of one loop iteration may take for granted: a phase
+ * function kind of every live lane without a rare parameter and no packet
+ * near its step limit, or (-1) nothing. */
+template <int KIND> struct RoundKind {
+    static constexpr int kind = KIND;
+};
 
 /* The per-step fields of a packet's current layer, kept in registers: top,
  * bottom, 1/mut and mua/mut (the first 16 bytes of the record) and the
- * phase-function parameters. */
-XO_DEV void layer_state(const LayerL &Q, float4 &lt, PfL &pf) {
+ * phase-function parameters of its kind: g and beta share registers with a
+ * table's first two. */
+struct LanePf {
+    float p0, p1, p2; /* g, beta, - or a, b, c */
+    uint32_t loff, lsize_m1;
+    XO_DEV PfL get() const { return PfL{p0, p1, p0, p1, p2, loff, lsize_m1}; }
+};
+
+XO_DEV void layer_state(const LayerL &Q, bool table, float4 &lt, LanePf &pf) {
     lt = *reinterpret_cast<const float4 *>(&Q);
-    pf = PfL{Q.g, Q.beta, Q.la, Q.lb, Q.lc, Q.loff, Q.lsize_m1};
+    pf = LanePf{table ? Q.la : Q.g, table ? Q.lb : Q.beta, Q.lc, Q.loff, Q.lsize_m1};
 }
 
-/* Pending events of the split transport step. */
-constexpr uint32_t kEvNone = 0, kEvInteraction = 1, kEvBoundary = 2;
-/* Boundary events are handled once P.defer_min lanes of the wave hold one,
- * or after kDeferWait iterations (bounded wait, every event is handled). */
+/* What a lane does next: draw a step, an interaction (only after a step that
+ * crossed both planes of a degenerate layer), a boundary event, or nothing
+ * (no packet). One register, tested once per round. */
+constexpr uint32_t kStep = 0, kInteraction = 1, kBoundary = 2, kIdle = 3;
+/* Boundary events are handled once P.defer_min of 64 live lanes of the wave
+ * hold one, or after kDeferWait iterations (bounded wait, every event is
+ * handled). */
 constexpr uint32_t kDeferWait = 8;
 /* Transport rounds (B then C) per loop iteration: 1.66e9 -> 1.92e9
  * packets/s on the 4096-instance batch going from 1 to 6 (2: 1.83e9, 3:
  * 1.89e9, 8: 1.93e9; ending the rounds early once a quarter of the lanes
- * wait: 1.86e9). */
-constexpr int kStepsPerIteration = 6;
+ * wait: 1.86e9). The rounds are compiled per phase-function kind and picked
+ * once per iteration for the whole wave (items come grouped by kind); what
+ * only rare parameters, a radius or the step limit need is tested there too,
+ * so that a step of Henyey-Greenstein is about 86 vector and 22 scalar
+ * instructions instead of 100 and 75. A wave running its last long packet
+ * waits for each of them: 64 instances of 1e3-1e5 packets 40 -> 27 ms. */
+constexpr uint32_t kStepsPerIteration = 6;
 
-/* End of an event (mcml.template.c:756-782): the simulation radius and the
- * step limit; a finished packet frees its lane and adds its steps to the
- * lane's count (every step ends in exactly one event). */
-__device__ __forceinline__ void end_event(bool done, bool &alive, float px, float py, float pz,
-                                          float spx, float spy, float spz, float rmax2,
-                                          uint32_t &pkt_steps, uint32_t *truncated,
-                                          uint32_t *steps) {
-    /* no distance can exceed an infinite radius (the default): skip the
-     * test, which changes nothing */
-    if (rmax2 < XO_INF_F) {
-        const float ex = px - spx, ey = py - spy, ez = pz - spz;
-        if (ex * ex + ey * ey + ez * ez > rmax2) done = true;
-    }
-    ++pkt_steps;
-    if (!done && pkt_steps >= XO_MAX_PACKET_STEPS) {
-        done = true;
-        atomicAdd(truncated, 1u);
-    }
-    if (done) {
-        alive = false;
-        atomicAdd(steps, pkt_steps);
-    }
-}
-
-/* At most 64 VGPRs (8 waves per SIMD): the compiler fits the loop without
- * spills, and the extra wave hides more of the layer and LUT reads (+2.5 %
- * packets/s over 72 VGPRs and 7 waves). METHOD is the stepping method of
+/* Seven waves per SIMD (72 VGPRs): the loop holds a copy of its rounds per
+ * phase-function kind, and at eight waves (64) the registers it spills cost
+ * more than the wave hides (2000-instance batch, hardware arithmetic: 285 ms
+ * at eight, 277 at seven, 295 at six). METHOD is the stepping method of
  * every instance (xo_method), M the arithmetic (MathExact, MathFast), FLU
  * whether any instance has a fluence grid. */
 template <int METHOD, class M, bool FLU>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7)))
 batch_kernel(const BatchParams P) {
     __shared__ BatchBlockStats sstats;
-    /* per-thread event counts in LDS (packets, steps, boundary events,
+    /* per thread, in LDS: event counts (packets, steps, boundary events,
      * truncated packets and, with fluence grids, deposits), added with LDS
-     * atomics: kept in registers they would take four or five of the
-     * loop's 64 */
-    constexpr int kCounts = FLU ? 5 : 4;
-    __shared__ uint32_t scount[kCounts][256];
-    for (int k = 0; k < kCounts; ++k) scount[k][threadIdx.x] = 0u;
+     * atomics, and the simulation sphere of its packet (source position and
+     * squared radius), read only where some packet of the wave has a finite
+     * one: kept in registers they would take eight of the loop's 64 */
+    extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
+    constexpr uint32_t kCounts = FLU ? 5 : 4;
+    const uint32_t nthreads = blockDim.x;
+    uint32_t *const scount = smem + threadIdx.x;
+    float4 *const sphere = reinterpret_cast<float4 *>(smem + kCounts * nthreads) + threadIdx.x;
+    for (uint32_t k = 0; k < kCounts; ++k) scount[k * nthreads] = 0u;
+    auto count = [&](uint32_t k, uint32_t n) { atomicAdd(&scount[k * nthreads], n); };
     if (threadIdx.x < XO_STAT_COUNT) sstats.v[threadIdx.x] = 0ull;
     __syncthreads();
     const uint32_t nitems = P.nitems_ptr ? *P.nitems_ptr : P.nitems;
@@ -110,11 +114,9 @@ batch_kernel(const BatchParams P) {
     bool queue_empty = false;
 
     /* lane state */
-    bool alive = false;
+    uint32_t state = kIdle;
     uint32_t inst = 0;
-    const LayerL *layers = P.layers;
-    int32_t nl = 3, pf_kind = 0;
-    float rmax2 = 0.f, spx = 0.f, spy = 0.f, spz = 0.f;
+    int32_t pf_kind = 0;
     float px = 0.f, py = 0.f, pz = 0.f, dx = 0.f, dy = 0.f, dz = 0.f, w = 0.f;
     int32_t layer = 1;
     uint64_t x = 0;
@@ -125,21 +127,22 @@ batch_kernel(const BatchParams P) {
      * event), not in every step (+14 % packets/s; the compiler spills a
      * few rarely used registers to stay at 64) */
     float4 lt = make_float4(0.f, 0.f, 0.f, 0.f);
-    PfL lpf{0.f, 0.f, 0.f, 0.f, 0.f, 0u, 0u};
-    uint32_t *const n_trunc = &scount[3][threadIdx.x];
-    uint32_t *const n_steps = &scount[1][threadIdx.x];
-    uint32_t pend = kEvNone;  /* event the lane's last step ended on     */
+    LanePf lpf{0.f, 0.f, 0.f, 0u, 0u};
+    auto layer_of = [&](int32_t l) -> const LayerL & {
+        return P.layers[(size_t)inst * XO_BATCH_MAX_LAYERS + (uint32_t)l];
+    };
     float pstep = 0.f;        /* drawn step of a pending boundary event  */
     uint32_t bwait = 0;       /* iterations boundary events have waited  */
+    bool finite = false;      /* the packet's simulation radius is       */
 
     for (;;) {
         /* ---- hand out packets to the lanes that need one, once at least
          * refill_min of them (or every lane) wait: one refill serves many
          * lanes, the rest of the time no lane runs the launch code ---- */
-        const bool want = !alive && !queue_empty;
+        const bool want = state == kIdle && !queue_empty;
         const uint64_t m = __ballot(want);
         const uint32_t nwant = (uint32_t)__builtin_popcountll(m);
-        const uint32_t nalive = (uint32_t)__builtin_popcountll(__ballot(alive));
+        const uint32_t nalive = (uint32_t)__builtin_popcountll(__ballot(state != kIdle));
         const uint32_t rank = prefix_count(m);
         uint32_t assigned = 0;
         bool launch = false;
@@ -181,16 +184,12 @@ batch_kernel(const BatchParams P) {
         }
         if (launch) {
             const BatchHdr &H = P.hdr[inst];
-            layers = P.layers + (size_t)inst * XO_BATCH_MAX_LAYERS;
-            nl = H.num_layers;
             pf_kind = H.pf_kind;
-            rmax2 = H.rmax2;
-            spx = H.src_pos[0];
-            spy = H.src_pos[1];
-            spz = H.src_pos[2];
+            *sphere = make_float4(H.src_pos[0], H.src_pos[1], H.src_pos[2], H.rmax2);
+            finite = H.rmax2 < XO_INF_F;
             xo_packet_state(H.seed, my_p, P.table, &x, &a);
             if (H.src_kind == XO_SRC_FIBER_NI) {
-                const float n1 = layers[1].n;
+                const float n1 = layer_of(1).n;
                 const float R =
                     fiber_ni_launch<M>(H.fiber, n1, x, a, px, py, pz, dx, dy, dz, w);
                 if (H.specular.kind != XO_DET_NONE) {
@@ -200,30 +199,57 @@ batch_kernel(const BatchParams P) {
                 }
             } else if (H.src_kind == XO_SRC_FIBER) {
                 /* UniformFiber, xopto/mcml/mcsource/fiber.py:265-330 */
-                const float R = fiber_launch<M>(H.fiber, H.fiber_axis, layers[1].n, x, a, px,
+                const float R = fiber_launch<M>(H.fiber, H.fiber_axis, layer_of(1).n, x, a, px,
                                                 py, pz, dx, dy, dz, w);
                 detector_deposit<M>(H.specular, bins, px, py, dx, dy, dz, R);
             } else {
                 /* Line source, xopto/mcml/mcsource/line.py:95-110 */
                 w = 1.0f - H.reflectance;
-                px = spx;
-                py = spy;
-                pz = spz;
+                px = H.src_pos[0];
+                py = H.src_pos[1];
+                pz = H.src_pos[2];
                 dx = H.dir_sample[0];
                 dy = H.dir_sample[1];
                 dz = H.dir_sample[2];
             }
             layer = 1;
-            layer_state(layers[1], lt, lpf);
+            layer_state(layer_of(1), pf_kind == XO_PF_LUT, lt, lpf);
+            /* the steps of the lane's last packet (every step ends in
+             * exactly one event) */
+            count(1, pkt_steps);
             pkt_steps = 0;
-            alive = true;
-            atomicAdd(&scount[0][threadIdx.x], 1u);
+            state = kStep;
+            count(0, 1u);
         }
-        if (!__any(alive)) {
+        if (!__any(state != kIdle)) {
             if (queue_empty) break;
             continue;
         }
-        if (!alive) continue;
+        /* whether this iteration handles the boundary events (A below);
+         * taken by every lane, so that the wait count stays uniform */
+        const uint32_t nb = (uint32_t)__builtin_popcountll(__ballot(state == kBoundary));
+        const uint32_t nal = (uint32_t)__builtin_popcountll(__ballot(state != kIdle));
+        const bool run_b =
+            nb != 0 && (64u * nb >= P.defer_min * nal || nb == nal || bwait >= kDeferWait);
+        bwait = (nb != 0 && !run_b) ? bwait + 1u : 0u;
+        const bool any_rmax = __any(state != kIdle && finite);
+        if (state == kIdle) continue;
+        /* end of an event (mcml.template.c:756-782): the simulation radius
+         * and the step limit. No distance exceeds an infinite radius (the
+         * default): without a finite one in the wave the test is left out. */
+        auto end_event = [&](bool done, bool limit) {
+            if (any_rmax) {
+                const float4 sp = *sphere;
+                const float ex = px - sp.x, ey = py - sp.y, ez = pz - sp.z;
+                done = done || ex * ex + ey * ey + ez * ez > sp.w;
+            }
+            ++pkt_steps;
+            if (limit && !done && pkt_steps >= XO_MAX_PACKET_STEPS) {
+                done = true;
+                count(3, 1u);
+            }
+            state = done ? kIdle : kStep;
+        };
 
         /* an instance's fluence deposit (fluence.py:102-147); the grid is
          * read from the instance header only when the batch has one */
@@ -231,7 +257,7 @@ batch_kernel(const BatchParams P) {
             const FluenceL &F = P.hdr[inst].fluence;
             if (F.enabled != XO_FLUENCE_NONE &&
                 fluence_deposit<M>(F, P.accum, qx, qy, qz, deposit, mua))
-                atomicAdd(&scount[kCounts - 1][threadIdx.x], 1u);
+                count(kCounts - 1, 1u);
         };
         /* microscopic Beer-Lambert: absorption along the whole step
          * (mcml.template.c:584-606); with a fluence grid the deposit goes
@@ -259,29 +285,21 @@ batch_kernel(const BatchParams P) {
         };
 
         /* ---- transport steps, mcml.template.c:514-788, in three phases
-         * per iteration. (B) lanes without a pending event draw a step; a
-         * step that stays inside the layer moves the packet and leaves an
-         * interaction event, a step that reaches a layer boundary is kept
-         * pending. (C) every interaction event is handled. (A, at the start
-         * of the next iterations) boundary events, a few percent of the
-         * steps in turbid layers, are handled together once defer_min lanes
-         * of the wave hold one, every alive lane holds one, or they waited
-         * kDeferWait iterations: the clipping of the step to the boundary,
-         * the move and the Fresnel event then run for those lanes only,
-         * instead of in nearly every iteration for two or three lanes.
-         * Each packet's arithmetic and draws are those of the reference's
-         * loop; only when the wave issues them changes. ---- */
+         * per iteration. (B) lanes draw a step; a step that stays inside the
+         * layer moves the packet and (C) interacts, a step that reaches a
+         * layer boundary is kept pending. (A, at the start of the next
+         * iterations) boundary events, a few percent of the steps in turbid
+         * layers, are handled together once defer_min of 64 live lanes of
+         * the wave hold one or they waited kDeferWait iterations: the
+         * clipping of the step to the boundary, the move and the Fresnel
+         * event then run for those lanes only, instead of in nearly every
+         * iteration for two or three lanes. Each packet's arithmetic and
+         * draws are those of the reference's loop; only when the wave issues
+         * them changes. ---- */
         {
-            const uint32_t nb = (uint32_t)__builtin_popcountll(__ballot(pend == kEvBoundary));
-            const uint32_t nal = (uint32_t)__builtin_popcountll(__ballot(true));
-            /* the wait count of the first active lane (lanes that were idle
-             * hold stale counts), so the decision is wave-uniform */
-            const uint32_t bw = (uint32_t)__builtin_amdgcn_readfirstlane((int)bwait);
-            const bool run_b = nb != 0 && (64u * nb >= P.defer_min * nal || nb == nal || bw >= kDeferWait);
-            bwait = (nb != 0 && !run_b) ? bw + 1u : 0u;
-            if (run_b && pend == kEvBoundary) {
+            if (run_b && state == kBoundary) {
                 /* (A) the step as drawn, clipped to the boundary it reaches */
-                const LayerL L = layers[layer];
+                const LayerL L = layer_of(layer);
                 float step = pstep;
                 int32_t next = layer;
                 if (__builtin_fmaf(step, dz, pz) < L.top) {
@@ -299,11 +317,11 @@ batch_kernel(const BatchParams P) {
                 if (layer > next) pz = L.top;
                 if (METHOD == XO_METHOD_MBL) mbl_absorb(L, step);
                 if (next != layer) {
-                    atomicAdd(&scount[2][threadIdx.x], 1u);
-                    mcml_boundary<M>(layers, layer, next, dx, dy, dz, x, a);
+                    count(2, 1u);
+                    mcml_boundary<M>(&layer_of(0), layer, next, dx, dy, dz, x, a);
                     bool done = false;
-                    if (!(layer > 0 && layer < nl - 1)) {
-                        const BatchHdr &H = P.hdr[inst];
+                    const BatchHdr &H = P.hdr[inst];
+                    if (!(layer > 0 && layer < H.num_layers - 1)) {
                         if (layer <= 0)
                             detector_deposit<M>(H.top, bins, px, py, dx, dy, dz, w);
                         else
@@ -311,97 +329,117 @@ batch_kernel(const BatchParams P) {
                         done = true;
                     }
                     done = mbl_roulette(done);
-                    pend = kEvNone;
-                    layer_state(layers[layer], lt, lpf);
-                    end_event(done, alive, px, py, pz, spx, spy, spz, rmax2, pkt_steps, n_trunc,
-                              n_steps);
+                    layer_state(layer_of(layer), pf_kind == XO_PF_LUT, lt, lpf);
+                    end_event(done, true);
                 } else {
                     /* crossed both planes of a degenerate layer: an
-                     * interaction at the clipped point, handled below */
-                    pend = kEvInteraction;
+                     * interaction at the clipped point */
+                    state = kInteraction;
                 }
             }
         }
+        /* (C) absorption and scattering, mcml.template.c:696-753 */
+        auto interact = [&](auto rk) {
+            constexpr int K = decltype(rk)::kind;
+            bool done = false;
+            if (METHOD == XO_METHOD_AR && rng_next(x, a) < lt.w) {
+                /* albedo rejection: the whole weight is absorbed here */
+                if (FLU) fluence_at(px, py, pz, w, layer_of(layer).mua);
+                w = 0.0f;
+                done = true;
+            } else {
+                if (METHOD == XO_METHOD_AW) {
+                    float deposit = w * lt.w;
+                    w -= deposit;
+                    if (FLU) fluence_at(px, py, pz, deposit, layer_of(layer).mua);
+                }
+                float xi_fi, ct;
+                if constexpr (K < 0)
+                    ct = pf_sample_rt<M>(pf_kind, lpf.get(), P.lut, x, a, xi_fi);
+                else
+                    ct = pf_sample<K, false, M>(lpf.get(), P.lut, x, a, xi_fi);
+                scatter_direction<M>(dx, dy, dz, ct, xi_fi);
+                if (METHOD == XO_METHOD_AW)
+                    done = roulette(w, x, a, P.w_min, P.chance, P.use_lottery);
+            }
+            done = mbl_roulette(done);
+            end_event(done, K < 0);
+        };
         /* (B) and (C) kStepsPerIteration times per iteration: the loop-top
          * work (refill and boundary ballots, the wave-uniform decisions)
          * is shared by that many steps; a lane whose packet ends or whose
          * step reaches a boundary sits out the remaining rounds */
-#pragma unroll
-        for (int rep = 0; rep < kStepsPerIteration; ++rep) {
-            if (alive && pend == kEvNone) {
-                /* (B) */
+        auto round = [&](auto rk) {
+            bool inside = state == kStep;
+            if (inside) {
                 float step;
                 if (METHOD == XO_METHOD_MBL)
                     step = M::div(-M::log_unit(rng_next(x, a)),
-                                  layers[layer].mus); /* mcml.template.c:529-531 */
+                                  layer_of(layer).mus); /* mcml.template.c:529-531 */
                 else
                     step = -M::log_unit(rng_next(x, a)) * lt.z;
                 step = fminf(step, XO_FLT_MAX);
                 const float zend = __builtin_fmaf(step, dz, pz);
+                pstep = step;
                 if (zend < lt.x || zend >= lt.y) {
-                    pend = kEvBoundary;
-                    pstep = step;
+                    state = kBoundary;
+                    inside = false;
                 } else {
                     px = __builtin_fmaf(dx, step, px);
                     py = __builtin_fmaf(dy, step, py);
                     pz = zend;
-                    if (METHOD == XO_METHOD_MBL) mbl_absorb(layers[layer], step);
-                    pend = kEvInteraction;
+                    if (METHOD == XO_METHOD_MBL) mbl_absorb(layer_of(layer), step);
                 }
             }
-            if (alive && pend == kEvInteraction) {
-                /* (C) absorption and scattering, mcml.template.c:696-753 */
-                const LayerL &L = layers[layer];
-                bool done = false;
-                if (METHOD == XO_METHOD_AR && rng_next(x, a) < lt.w) {
-                    /* albedo rejection: the whole weight is absorbed here */
-                    if (FLU) fluence_at(px, py, pz, w, L.mua);
-                    w = 0.0f;
-                    done = true;
-                } else {
-                    if (METHOD == XO_METHOD_AW) {
-                        float deposit = w * lt.w;
-                        w -= deposit;
-                        if (FLU) fluence_at(px, py, pz, deposit, L.mua);
-                    }
-                    float xi_fi;
-                    float ct = pf_sample_rt<M>(pf_kind, lpf, P.lut, x, a, xi_fi);
-                    scatter_direction<M>(dx, dy, dz, ct, xi_fi);
-                    if (METHOD == XO_METHOD_AW)
-                        done = roulette(w, x, a, P.w_min, P.chance, P.use_lottery);
-                }
-                done = mbl_roulette(done);
-                pend = kEvNone;
-                end_event(done, alive, px, py, pz, spx, spy, spz, rmax2, pkt_steps, n_trunc,
-                          n_steps);
-            }
-        }
+            if (inside || (decltype(rk)::kind < 0 && state == kInteraction)) interact(rk);
+        };
+        auto rounds = [&](auto rk) {
+#pragma unroll
+            for (uint32_t rep = 0; rep < kStepsPerIteration; ++rep) round(rk);
+        };
+        const int kind = __builtin_amdgcn_readfirstlane(pf_kind);
+        if (__any(state == kInteraction || pf_kind != kind || pf_rare<M>(pf_kind, lpf.get()) ||
+                  pkt_steps >= XO_MAX_PACKET_STEPS - kStepsPerIteration))
+#pragma unroll 1
+            for (uint32_t rep = 0; rep < kStepsPerIteration; ++rep) round(RoundKind<-1>{});
+        else if (kind == XO_PF_HG)
+            rounds(RoundKind<XO_PF_HG>{});
+        else if (kind == XO_PF_MHG)
+            rounds(RoundKind<XO_PF_MHG>{});
+        else
+            rounds(RoundKind<XO_PF_LUT>{});
     }
+    count(1, pkt_steps);
 
     const int kinds[5] = {XO_STAT_PACKETS, XO_STAT_STEPS, XO_STAT_BOUNDARY, XO_STAT_TRUNCATED,
                           XO_STAT_DEPOSITS};
-    for (int k = 0; k < kCounts; ++k)
-        if (scount[k][threadIdx.x])
-            atomicAdd(&sstats.v[kinds[k]], (unsigned long long)scount[k][threadIdx.x]);
+    for (uint32_t k = 0; k < kCounts; ++k)
+        if (scount[k * nthreads])
+            atomicAdd(&sstats.v[kinds[k]], (unsigned long long)scount[k * nthreads]);
     __syncthreads();
     if (threadIdx.x < XO_STAT_COUNT && sstats.v[threadIdx.x])
         atomicAdd(&P.stats[threadIdx.x], sstats.v[threadIdx.x]);
 }
 
+static size_t batch_lds_bytes(uint32_t block, bool fluence) {
+    return (size_t)block * 4u * (4u + (fluence ? 5u : 4u));
+}
+
 template <class M, bool FLU>
 static hipError_t launch_batch_m(const BatchParams &P, uint32_t blocks, uint32_t block,
                                  hipStream_t stream) {
+    const size_t lds = batch_lds_bytes(block, FLU);
     switch (P.method) {
     case XO_METHOD_AW:
-        hipLaunchKernelGGL((batch_kernel<XO_METHOD_AW, M, FLU>), dim3(blocks), dim3(block), 0,
+        hipLaunchKernelGGL((batch_kernel<XO_METHOD_AW, M, FLU>), dim3(blocks), dim3(block), lds,
                            stream, P);
         break;
     case XO_METHOD_AR:
-        hipLaunchKernelGGL((batch_kernel<XO_METHOD_AR, M, FLU>), dim3(blocks), dim3(block), 0,
+        hipLaunchKernelGGL((batch_kernel<XO_METHOD_AR, M, FLU>), dim3(blocks), dim3(block), lds,
                            stream, P);
         break;
     case XO_METHOD_MBL:
-        hipLaunchKernelGGL((batch_kernel<XO_METHOD_MBL, M, FLU>), dim3(blocks), dim3(block), 0,
+        hipLaunchKernelGGL((batch_kernel<XO_METHOD_MBL, M, FLU>), dim3(blocks), dim3(block), lds,
                            stream, P);
         break;
     default:
@@ -435,7 +473,8 @@ hipError_t launch_zero_u32(uint32_t *ptr, uint32_t n, hipStream_t stream) {
 hipError_t occupancy_batch(uint32_t block, int *blocks_per_cu) {
     /* the albedo-weight build stands for all three methods */
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        blocks_per_cu, batch_kernel<XO_METHOD_AW, MathExact, false>, (int)block, 0);
+        blocks_per_cu, batch_kernel<XO_METHOD_AW, MathExact, false>, (int)block,
+        batch_lds_bytes(block, true));
 }
 
 } // namespace xo

@@ -61,16 +61,13 @@ XO_DEV float sqrt_in_range(float x) {
     return r;
 }
 
-/* Correctly rounded a / b for normal a, b with 2^-60 <= |a|, |b| <= 2^60:
- * reciprocal estimate, one Newton step on it, quotient, two residual
- * corrections (the compiler's general division sequence without the
- * operand scaling and the special-case fix-up, which leave such operands
- * unchanged). Checked against the division on 2^32 random operand pairs of
- * that range. Callers: 1 / |d| for a direction d of length about 1. */
-XO_DEV float div_in_range(float a, float b) {
-    float y = __builtin_amdgcn_rcpf(b);
-    const float e = __builtin_fmaf(-b, y, 1.0f);
-    y = __builtin_fmaf(e, y, y);
+/* The refined reciprocal of b that div_in_range starts from, and the rest of
+ * that division: quotients by the same b share it. */
+XO_DEV float rcp_in_range(float b) {
+    const float y = __builtin_amdgcn_rcpf(b);
+    return __builtin_fmaf(__builtin_fmaf(-b, y, 1.0f), y, y);
+}
+XO_DEV float div_with_rcp(float a, float b, float y) {
     float q = a * y;
     float r = __builtin_fmaf(-b, q, a);
     q = __builtin_fmaf(r, y, q);
@@ -78,12 +75,14 @@ XO_DEV float div_in_range(float a, float b) {
     return __builtin_fmaf(r, y, q);
 }
 
-/* a / k for k = sqrt(1 - c^2) with |c| < 1 (so 2^-12 < k <= 1) and |a| <= 2:
- * the range-restricted division when |a| >= 2^-60, the general one for
- * smaller |a| (rare; it keeps the sign of a zero). Same bits either way. */
-XO_DEV float div_by_k(float a, float k) {
-    if (__builtin_expect(fabsf(a) >= 0x1p-60f, 1)) return div_in_range(a, k);
-    return a / k;
+/* Correctly rounded a / b for normal a, b with 2^-60 <= |a|, |b| <= 2^60:
+ * reciprocal estimate, one Newton step on it, quotient, two residual
+ * corrections (the compiler's general division sequence without the
+ * operand scaling and the special-case fix-up, which leave such operands
+ * unchanged). Checked against the division on 2^32 random operand pairs of
+ * that range. Callers: 1 / |d| for a direction d of length about 1. */
+XO_DEV float div_in_range(float a, float b) {
+    return div_with_rcp(a, b, rcp_in_range(b));
 }
 
 /* Arithmetic of the transport step, a template parameter of the kernels.
@@ -110,11 +109,23 @@ struct MathExact {
     XO_DEV static void sincos_turns(float t, float *s, float *c) { xo_sincos_turns(t, s, c); }
     XO_DEV static float cbrt(float x) { return xo_cbrtf(x); }
     XO_DEV static float sqrt(float x) { return __builtin_sqrtf(x); }
-    /* the range-restricted forms (see sqrt_in_range, div_in_range,
-     * div_by_k for their ranges) */
+    /* the range-restricted forms (see sqrt_in_range, div_in_range) */
     XO_DEV static float sqrt_r(float x) { return sqrt_in_range(x); }
     XO_DEV static float div_r(float a, float b) { return div_in_range(a, b); }
-    XO_DEV static float div_k(float a, float k) { return div_by_k(a, k); }
+    /* a, b <- a / k, b / k for k = sqrt(1 - c^2) with |c| < 1 (so 2^-12 < k
+     * <= 1) and |a|, |b| <= 2: the range-restricted division above 2^-60, the
+     * general one below (rare; it keeps the sign of a zero), so the same
+     * bits. Where `unused` (k may be 0) the results do not matter. */
+    XO_DEV static void div2_k(float &a, float &b, float k, bool unused) {
+        const float y = rcp_in_range(k);
+        float qa = div_with_rcp(a, k, y), qb = div_with_rcp(b, k, y);
+        if (__builtin_expect(fminf(fabsf(a), fabsf(b)) < 0x1p-60f && !unused, 0)) {
+            if (fabsf(a) < 0x1p-60f) qa = a / k;
+            if (fabsf(b) < 0x1p-60f) qb = b / k;
+        }
+        a = qa;
+        b = qb;
+    }
     /* 1 / sqrt(x) for the squared norm x of a near-unit vector */
     XO_DEV static float rsqrt_r(float x) { return div_in_range(1.0f, sqrt_in_range(x)); }
     XO_DEV static float div(float a, float b) { return a / b; }
@@ -140,7 +151,11 @@ struct MathFast {
     XO_DEV static float sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
     XO_DEV static float sqrt_r(float x) { return __builtin_amdgcn_sqrtf(x); }
     XO_DEV static float div_r(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-    XO_DEV static float div_k(float a, float k) { return a * __builtin_amdgcn_rcpf(k); }
+    XO_DEV static void div2_k(float &a, float &b, float k, bool) {
+        const float y = __builtin_amdgcn_rcpf(k);
+        a *= y;
+        b *= y;
+    }
     XO_DEV static float rsqrt_r(float x) { return __builtin_amdgcn_rsqf(x); }
     XO_DEV static float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 };
@@ -432,49 +447,67 @@ struct PfL {
     uint32_t loff, lsize_m1;
 };
 
+/* Whether a phase function needs the general sampling code (pf_sample with
+ * RARE): |g| so small that 2 g leaves the range of the short division (0
+ * among it, which draws once more), or table parameters for which the index
+ * division may. A property of the layer, tested where the layer may change;
+ * the steps between then skip the tests. */
+template <class M> __host__ __device__ inline bool pf_rare(int kind, const PfL &pf) {
+    if (kind != XO_PF_LUT) return !(fabsf(pf.g) >= 0x1p-60f);
+    if (M::fast) return false;
+    /* the divisor xi - c, 0 <= xi <= 1, keeps |c| or |c - 1| from 0 */
+    return !(fabsf(pf.la) >= 0x1p-60f && fabsf(pf.la) <= 0x1p60f &&
+             (pf.lc <= -0x1p-60f || pf.lc > 1.0f) && fabsf(pf.lc) <= 0x1p59f);
+}
+
 /* mcsim_pf_sample_angles: returns cos(theta), the azimuth as a fraction of
  * a turn in xi_fi. HG hg.py:80-96; MHg mhg.py:87-109; Lut lut.py:125-150
- * (index clamped to the table). */
-template <int PF, class M = MathExact>
+ * (index clamped to the table). RARE: for any parameters, else for those
+ * that pf_rare lets through (the same bits). */
+template <int PF, bool RARE, class M = MathExact>
 XO_DEV float pf_sample(const PfL &pf, const float *lut, uint64_t &x, uint32_t a,
                        float &xi_fi) {
     xi_fi = rng_next(x, a);
-    if constexpr (PF == XO_PF_HG) {
-        float g = pf.g;
+    auto hg = [&]() {
         /* |g| <= 1 (the host clips it): the numerator is +0 or >= 2^-24, the
          * denominator 0 or in [2^-24, 2]; a 0 denominator gives NaN either
          * way, which the clamp below turns into the same cosine */
-        float k = M::div_r(1.0f - g * g, 1.0f + g * (2.0f * rng_next(x, a) - 1.0f));
-        float ct = M::div(1.0f + g * g - k * k, 2.0f * g);
+        const float g = pf.g;
+        const float k = M::div_r(1.0f - g * g, 1.0f + g * (2.0f * rng_next(x, a) - 1.0f));
+        const float num = 1.0f + g * g - k * k; /* +0 or |num| >= 2^-24 */
+        if (!RARE) return M::div_r(num, 2.0f * g);
+        float ct = M::div(num, 2.0f * g);
         if (g == 0.0f) ct = 1.0f - 2.0f * rng_next(x, a);
+        return ct;
+    };
+    if constexpr (PF == XO_PF_HG) {
+        const float ct = hg();
         return fmaxf(fminf(ct, 1.0f), -1.0f);
     } else if constexpr (PF == XO_PF_MHG) {
-        float g = pf.g;
         float ct;
-        if (rng_next(x, a) <= pf.beta) {
-            /* as for Hg: |g| <= 1 */
-            float k = M::div_r(1.0f - g * g, 1.0f + g * (2.0f * rng_next(x, a) - 1.0f));
-            ct = M::div(1.0f + g * g - k * k, 2.0f * g);
-            if (g == 0.0f) ct = 1.0f - 2.0f * rng_next(x, a);
-        } else {
+        if (rng_next(x, a) <= pf.beta)
+            ct = hg();
+        else
             ct = M::cbrt(2.0f * rng_next(x, a) - 1.0f);
-        }
         return fminf(fmaxf(ct, -1.0f), 1.0f);
     } else {
-        float fsize = (float)pf.lsize_m1;
-        float fi = (M::div(pf.la, rng_next(x, a) - pf.lc) - pf.lb + 1.0f) * fsize *
+        const float fsize = (float)pf.lsize_m1;
+        const float den = rng_next(x, a) - pf.lc;
+        float fi = ((RARE ? M::div(pf.la, den) : M::div_r(pf.la, den)) - pf.lb + 1.0f) * fsize *
                    0.5f;
         fi = fminf(fmaxf(fi, 0.0f), fsize);
-        float fl = floorf(fi);
-        float d = fi - fl;
-        uint32_t i0 = (uint32_t)f2i_sat(fl);
-        uint32_t i1 = i0 + 1u < pf.lsize_m1 ? i0 + 1u : pf.lsize_m1;
+        const float fl = floorf(fi);
+        const float d = fi - fl;
+        const uint32_t i0 = (uint32_t)fl;
+        const uint32_t i1 = i0 + 1u < pf.lsize_m1 ? i0 + 1u : pf.lsize_m1;
         return lut[pf.loff + i0] * (1.0f - d) + lut[pf.loff + i1] * d;
     }
 }
 
 /* scatter_direction (mcbase.template.c:1522-1556) with the single-precision
- * renormalization (mc_normalize_fpv3, :975-981). */
+ * renormalization (mc_normalize_fpv3, :975-981). A direction along the axis
+ * has a form of its own, chosen after the other one has run for every lane:
+ * three selects instead of two branches. */
 template <class M = MathExact>
 XO_DEV void scatter_direction(float &dx, float &dy, float &dz, float ct,
                               float xi_fi) {
@@ -484,16 +517,17 @@ XO_DEV void scatter_direction(float &dx, float &dy, float &dz, float ct,
     float stcf = st * cos_fi;
     float stsf = st * sin_fi;
     float px = dx, py = dy, pz = dz;
-    if (fabsf(pz) >= kCos0) {
-        dx = stcf;
-        dy = stsf;
-        dz = copysignf(ct, pz * ct);
-    } else {
-        float k = M::sqrt_r(1.0f - pz * pz);
-        dx = M::div_k(stcf * px * pz - stsf * py, k) + px * ct;
-        dy = M::div_k(stcf * py * pz + stsf * px, k) + py * ct;
-        dz = (-stcf) * k + pz * ct;
-    }
+    const bool axial = fabsf(pz) >= kCos0;
+    float k = M::sqrt_r(1.0f - pz * pz);
+    dx = stcf * px * pz - stsf * py;
+    dy = stcf * py * pz + stsf * px;
+    M::div2_k(dx, dy, k, axial);
+    dx += px * ct;
+    dy += py * ct;
+    dz = (-stcf) * k + pz * ct;
+    dx = axial ? stcf : dx;
+    dy = axial ? stsf : dy;
+    dz = axial ? copysignf(ct, pz * ct) : dz;
     float inv = M::rsqrt_r(dx * dx + dy * dy + dz * dz);
     dx = dx * inv;
     dy = dy * inv;

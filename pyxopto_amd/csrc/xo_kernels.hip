@@ -396,7 +396,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
                             st[XO_STAT_DEPOSITS]++;
                     }
                     float xi_fi;
-                    float ct = pf_sample<PF, M>(lpf, lut, x, a, xi_fi);
+                    float ct = pf_sample<PF, true, M>(lpf, lut, x, a, xi_fi);
                     scatter_direction<M>(dx, dy, dz, ct, xi_fi);
                     if (TRACE) ts.ev |= XO_EVENT_SCATTERING;
                     if (METHOD == XO_METHOD_AW && roulette(w, x, a, w_min, chance, use_lottery))
@@ -779,7 +779,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
                 }
                 PfL pf{Mt.g, Mt.beta, Mt.la, Mt.lb, Mt.lc, Mt.loff, Mt.lsize_m1};
                 float xi_fi;
-                float ct = pf_sample<PF, M>(pf, lut, x, a, xi_fi);
+                float ct = pf_sample<PF, true, M>(pf, lut, x, a, xi_fi);
                 scatter_direction<M>(d[0], d[1], d[2], ct, xi_fi);
                 if (TRACE) ts.ev |= XO_EVENT_SCATTERING;
                 if (METHOD == XO_METHOD_AW && roulette(w, x, a, w_min, chance, use_lottery))
