@@ -460,6 +460,11 @@ template <class M> __host__ __device__ inline bool pf_rare(int kind, const PfL &
              (pf.lc <= -0x1p-60f || pf.lc > 1.0f) && fabsf(pf.lc) <= 0x1p59f);
 }
 
+/* Host: pf_rare of a packed phase function, for either arithmetic. */
+inline uint32_t pf_needs_rare(int kind, const xo_pf &f) {
+    return pf_rare<MathExact>(kind, PfL{f.g, f.beta, f.a, f.b, f.c, 0u, 0u}) ? 1u : 0u;
+}
+
 /* mcsim_pf_sample_angles: returns cos(theta), the azimuth as a fraction of
  * a turn in xi_fi. HG hg.py:80-96; MHg mhg.py:87-109; Lut lut.py:125-150
  * (index clamped to the table). RARE: for any parameters, else for those

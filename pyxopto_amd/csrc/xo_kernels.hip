@@ -14,6 +14,8 @@
  */
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "xo_device.h"
 #include "xo_kernels.h"
 #include "xo_seedhash.h"
@@ -29,22 +31,27 @@ struct BlockStats {
     unsigned long long v[XO_STAT_COUNT];
 };
 
-XO_DEV void stats_flush(BlockStats *ss, const uint32_t *mine,
-                        unsigned long long *gstats) {
-    for (int i = 0; i < XO_STAT_COUNT; ++i)
-        if (mine[i]) atomicAdd(&ss->v[i], (unsigned long long)mine[i]);
+/* Counts of events that are a few percent of the steps go to the block's
+ * counters in LDS as they happen; a lane keeps only those of every step. */
+XO_DEV void stat_add(BlockStats *ss, int kind, uint32_t n) {
+    if (n) atomicAdd(&ss->v[kind], (unsigned long long)n);
+}
+
+XO_DEV void stats_flush(BlockStats *ss, unsigned long long *gstats) {
     __syncthreads();
     if (threadIdx.x < XO_STAT_COUNT && ss->v[threadIdx.x])
         atomicAdd(&gstats[threadIdx.x], ss->v[threadIdx.x]);
 }
 
-/* Pending events of the split transport step of the layered kernel;
- * boundary events wait until kDeferMin lanes of a wave hold one (at most
- * kDeferWait iterations). */
-constexpr uint32_t kEvNone = 0, kEvInteraction = 1, kEvBoundary = 2;
+/* What a lane of the layered kernel does next: draw a step, an interaction
+ * (only after a step that crossed both planes of a degenerate layer), a
+ * boundary event, or nothing (no packet). Boundary events wait until
+ * kDeferMin of 64 live lanes of a wave hold one (at most kDeferWait
+ * iterations). */
+constexpr uint32_t kStep = 0, kInteraction = 1, kBoundary = 2, kIdle = 3;
 constexpr uint32_t kDeferMin = 12, kDeferWait = 8;
 /* Transport rounds (B then C) per loop iteration of the layered kernel. */
-constexpr int kRoundsPerIteration = 6;
+constexpr uint32_t kRoundsPerIteration = 6;
 
 /* FLU: built with the fluence deposit. Without it the loop keeps to 64-72
  * registers (7 waves per SIMD); traced runs have one build for both. */
@@ -135,14 +142,13 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
 
     bool active = lane_ok;
     WaveDispenser wq;
-    bool alive = false;
+    uint32_t state = kIdle;
     float px = 0.f, py = 0.f, pz = 0.f, dx = 0.f, dy = 0.f, dz = 0.f, w = 0.f;
     int32_t layer = 1;
-    uint32_t st[XO_STAT_COUNT] = {0, 0, 0, 0, 0, 0, 0};
+    uint32_t deposits = 0, launched = 0;
     uint32_t pkt_steps = 0;
     TraceState ts{0, 0, 0, 0.0f};
     const xo_trace &T = P.trace;
-    uint32_t pend = kEvNone; /* event the lane's last step ended on      */
     float pstep = 0.f;       /* drawn step of a pending boundary event   */
     uint32_t bwait = 0;      /* iterations boundary events have waited   */
     /* the per-step fields of the packet's current layer (top, bottom,
@@ -163,7 +169,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
 
     for (;;) {
         /* ---- refill lanes whose packet ended ---- */
-        bool want = active && !alive;
+        bool want = active && state == kIdle;
         bool launch = false;
         uint64_t pkt_index = 0;
         if (static_sched) {
@@ -179,7 +185,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
         } else {
             bool retire = false;
             uint64_t claimed = 0;
-            launch = dispense(wq, want, alive, P.counter, P.npackets, claim_size(P), kRefillMin,
+            launch = dispense(wq, want, state != kIdle, P.counter, P.npackets, claim_size(P), kRefillMin,
                               pkt_index, retire, claimed);
             if (retire) active = false;
             /* every Line packet deposits the same specular integer at the
@@ -229,9 +235,10 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
             }
             layer = 1;
             layer_state(sl[1]);
-            alive = true;
+            state = kStep;
+            stat_add(&sstats, XO_STAT_STEPS, pkt_steps); /* of the lane's last packet */
             pkt_steps = 0;
-            st[XO_STAT_PACKETS]++;
+            ++launched;
             if (TRACE) {
                 /* mcml.template.c:513-520, 791-810 */
                 ts = TraceState{pkt_index, 0u, XO_EVENT_LAUNCH, 0.0f};
@@ -239,19 +246,23 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
                     trace_event(T, P.trace_data, ts, px, py, pz, dx, dy, dz, w);
             }
         }
-        if (!__any(alive)) break;
-        if (!alive) continue;
+        if (!__any(state != kIdle)) break;
+        /* whether this iteration handles the boundary events (A below);
+         * taken by every lane, so that the wait count stays uniform */
+        const uint32_t nb = (uint32_t)__builtin_popcountll(__ballot(state == kBoundary));
+        const uint32_t nal = (uint32_t)__builtin_popcountll(__ballot(state != kIdle));
+        const bool run_b = nb != 0 && (64u * nb >= kDeferMin * nal || bwait >= kDeferWait);
+        bwait = (nb != 0 && !run_b) ? bwait + 1u : 0u;
+        if (state == kIdle) continue;
         /* ---- transport steps, the while(!done) loop of
-         * mcml.template.c:514-788, in three phases per iteration: (B)
-         * lanes without a pending event draw a step; a step inside the layer
-         * moves the packet (and, for microscopic Beer-Lambert, absorbs along
-         * it) and leaves an interaction event, a step reaching a boundary is
-         * kept pending; (C) interaction events are handled; (A, at the top
-         * of later iterations) boundary events are handled together once
-         * kDeferMin lanes of the wave hold one, every live lane holds one,
-         * or they waited kDeferWait iterations. Each packet's arithmetic and
-         * draws follow the reference's loop; only when the wave issues them
-         * changes. ---- */
+         * mcml.template.c:514-788, in three phases per iteration: (B) lanes
+         * draw a step; a step inside the layer moves the packet (and, for
+         * microscopic Beer-Lambert, absorbs along it) and (C) interacts, a
+         * step reaching a boundary is kept pending; (A, at the top of later
+         * iterations) boundary events are handled together once kDeferMin of
+         * 64 live lanes of the wave hold one or they waited kDeferWait
+         * iterations. Each packet's arithmetic and draws follow the
+         * reference's loop; only when the wave issues them changes. ---- */
         auto mbl_absorb = [&](const LayerL &L, float step) {
             /* absorption along the whole step, mcml.template.c:584-606 */
             const float mua = L.mua;
@@ -265,23 +276,26 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
                         ? step - M::div(-M::log_unit(1.0f - rng_next(x, a) * fraction), mua)
                         : 0.0f;
                 if (deposit_fluence(px - back * dx, py - back * dy, pz - back * dz, deposit, mua))
-                    st[XO_STAT_DEPOSITS]++;
+                    ++deposits;
             }
         };
-        auto end_step = [&](bool done) {
+        auto end_step = [&](bool done, bool limit) {
             /* microscopic Beer-Lambert: roulette after the boundary or the
              * scattering, whether or not the packet has left (as the
              * reference does, mcml.template.c:652-667) */
             if (METHOD == XO_METHOD_MBL && roulette(w, x, a, w_min, chance, use_lottery))
                 done = true;
-            float ex = px - spx, ey = py - spy, ez = pz - spz;
-            if (rmax2 < XO_INF_F && ex * ex + ey * ey + ez * ez > rmax2) {
-                done = true;
-                if (TRACE) ts.ev |= XO_EVENT_ESCAPED;
+            if (rmax2 < XO_INF_F) {
+                const float ex = px - spx, ey = py - spy, ez = pz - spz;
+                const bool out = ex * ex + ey * ey + ez * ez > rmax2;
+                done = done || out;
+                if (TRACE && out) ts.ev |= XO_EVENT_ESCAPED;
             }
-            if (!done && ++pkt_steps >= XO_MAX_PACKET_STEPS) {
+            /* every step ends in exactly one event */
+            ++pkt_steps;
+            if (limit && !done && pkt_steps >= XO_MAX_PACKET_STEPS) {
                 done = true;
-                st[XO_STAT_TRUNCATED]++;
+                stat_add(&sstats, XO_STAT_TRUNCATED, 1u);
             }
             if (TRACE) {
                 /* mcml.template.c:765-781 */
@@ -291,128 +305,132 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcml_kernel(const McmlParams P) 
                 ts.ev = 0u;
                 if (done) P.trace_n[ts.pkt] = (int32_t)ts.count;
             }
-            pend = kEvNone;
-            if (done) alive = false;
+            state = done ? kIdle : kStep;
         };
-        {
-            const uint32_t nb = (uint32_t)__builtin_popcountll(__ballot(pend == kEvBoundary));
-            const uint32_t nal = (uint32_t)__builtin_popcountll(__ballot(true));
-            const uint32_t bw = (uint32_t)__builtin_amdgcn_readfirstlane((int)bwait);
-            const bool run_b = nb != 0 && (64u * nb >= kDeferMin * nal || bw >= kDeferWait);
-            bwait = (nb != 0 && !run_b) ? bw + 1u : 0u;
-            if (run_b && pend == kEvBoundary) {
-                /* (A) the step as drawn, clipped to the boundary it reaches */
-                const LayerL &L = sl[layer];
-                float step = pstep;
-                int32_t next = layer;
-                if (__builtin_fmaf(step, dz, pz) < L.top) {
-                    --next;
-                    if (fabsf(dz) != 0.0f) step = M::div(L.top - pz, dz);
+        if (run_b && state == kBoundary) {
+            /* (A) the step as drawn, clipped to the boundary it reaches */
+            const LayerL &L = sl[layer];
+            float step = pstep;
+            int32_t next = layer;
+            if (__builtin_fmaf(step, dz, pz) < L.top) {
+                --next;
+                if (fabsf(dz) != 0.0f) step = M::div(L.top - pz, dz);
+            }
+            if (__builtin_fmaf(step, dz, pz) >= L.bottom) {
+                ++next;
+                if (fabsf(dz) != 0.0f) step = M::div(L.bottom - pz, dz);
+            }
+            px = __builtin_fmaf(dx, step, px);
+            py = __builtin_fmaf(dy, step, py);
+            pz = __builtin_fmaf(dz, step, pz);
+            /* optical path length, mcml.template.c:570-574 */
+            if (TRACE && T.plon) ts.pl += L.n * step;
+            if (layer < next) pz = L.bottom;
+            if (layer > next) pz = L.top;
+            if (METHOD == XO_METHOD_MBL) mbl_absorb(L, step);
+            if (next != layer) {
+                stat_add(&sstats, XO_STAT_BOUNDARY, 1u);
+                const int32_t before = layer;
+                mcml_boundary<M>(sl, layer, next, dx, dy, dz, x, a);
+                layer_state(sl[layer]);
+                if (TRACE)
+                    ts.ev |= XO_EVENT_BOUNDARY_HIT |
+                             (layer != before ? XO_EVENT_REFRACTION : XO_EVENT_REFLECTION);
+                bool done = false;
+                if (!(layer > 0 && layer < (int32_t)nl - 1)) {
+                    if (layer <= 0)
+                        detector_deposit<M>(lds_fresh(sev.top), bins, px, py, dx, dy, dz, w);
+                    else
+                        detector_deposit<M>(lds_fresh(sev.bottom), bins, px, py, dx, dy, dz, w);
+                    done = true;
                 }
-                if (__builtin_fmaf(step, dz, pz) >= L.bottom) {
-                    ++next;
-                    if (fabsf(dz) != 0.0f) step = M::div(L.bottom - pz, dz);
-                }
-                px = __builtin_fmaf(dx, step, px);
-                py = __builtin_fmaf(dy, step, py);
-                pz = __builtin_fmaf(dz, step, pz);
-                /* optical path length, mcml.template.c:570-574 */
-                if (TRACE && T.plon) ts.pl += L.n * step;
-                if (layer < next) pz = L.bottom;
-                if (layer > next) pz = L.top;
-                if (METHOD == XO_METHOD_MBL) mbl_absorb(L, step);
-                if (next != layer) {
-                    st[XO_STAT_BOUNDARY]++;
-                    const int32_t before = layer;
-                    mcml_boundary<M>(sl, layer, next, dx, dy, dz, x, a);
-                    layer_state(sl[layer]);
-                    if (TRACE)
-                        ts.ev |= XO_EVENT_BOUNDARY_HIT |
-                                 (layer != before ? XO_EVENT_REFRACTION : XO_EVENT_REFLECTION);
-                    bool done = false;
-                    if (!(layer > 0 && layer < (int32_t)nl - 1)) {
-                        if (layer <= 0)
-                            detector_deposit<M>(lds_fresh(sev.top), bins, px, py, dx, dy, dz, w);
-                        else
-                            detector_deposit<M>(lds_fresh(sev.bottom), bins, px, py, dx, dy, dz,
-                                                w);
-                        done = true;
-                    }
-                    end_step(done);
-                } else {
-                    /* crossed both planes of a degenerate layer: an
-                     * interaction at the clipped point, handled below */
-                    pend = kEvInteraction;
-                }
+                end_step(done, true);
+            } else {
+                /* crossed both planes of a degenerate layer: an
+                 * interaction at the clipped point */
+                state = kInteraction;
             }
         }
-        /* (B) and (C) kRoundsPerIteration times per iteration, as in the
-         * batch kernel: the loop-top work is shared by that many steps
-         * (1 mm slab 0.464 -> 0.403 ms per 1e6 packets) */
-#pragma unroll
-        for (int rep = 0; rep < kRoundsPerIteration; ++rep) {
-            if (alive && pend == kEvNone) {
-                /* (B) */
-                const LayerL &L = sl[layer];
-                st[XO_STAT_STEPS]++;
+        /* (C), RARE: for any phase-function parameters and with the step
+         * limit */
+        auto interact = [&](auto rare) {
+            constexpr bool RARE = decltype(rare)::value;
+            bool done = false;
+            if (METHOD == XO_METHOD_AR && rng_next(x, a) < lt.w) {
+                /* albedo rejection: the whole weight is absorbed here,
+                 * mcml.template.c:696-708 */
+                const float deposit = w;
+                w -= deposit;
+                if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
+                if (use_fluence && deposit_fluence(px, py, pz, deposit, sl[layer].mua))
+                    ++deposits;
+                done = true;
+            } else {
+                if (METHOD == XO_METHOD_AW) {
+                    const float deposit = w * lt.w;
+                    w -= deposit;
+                    if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
+                    if (use_fluence && deposit_fluence(px, py, pz, deposit, sl[layer].mua))
+                        ++deposits;
+                }
+                float xi_fi;
+                float ct = pf_sample<PF, RARE, M>(lpf, lut, x, a, xi_fi);
+                scatter_direction<M>(dx, dy, dz, ct, xi_fi);
+                if (TRACE) ts.ev |= XO_EVENT_SCATTERING;
+                if (METHOD == XO_METHOD_AW && roulette(w, x, a, w_min, chance, use_lottery))
+                    done = true;
+            }
+            end_step(done, RARE);
+        };
+        /* (B) and (C) */
+        auto round = [&](auto rare) {
+            constexpr bool RARE = decltype(rare)::value;
+            bool inside = state == kStep;
+            if (inside) {
                 float step;
                 if (METHOD == XO_METHOD_MBL)
-                    step = M::div(-M::log_unit(rng_next(x, a)), L.mus); /* mcml.template.c:529-531 */
+                    step = M::div(-M::log_unit(rng_next(x, a)),
+                                  sl[layer].mus); /* mcml.template.c:529-531 */
                 else
                     step = -M::log_unit(rng_next(x, a)) * lt.z;
                 step = fminf(step, XO_FLT_MAX);
                 const float zend = __builtin_fmaf(step, dz, pz);
+                pstep = step;
                 if (zend < lt.x || zend >= lt.y) {
-                    pend = kEvBoundary;
-                    pstep = step;
+                    state = kBoundary;
+                    inside = false;
                 } else {
                     px = __builtin_fmaf(dx, step, px);
                     py = __builtin_fmaf(dy, step, py);
                     pz = zend;
-                    if (TRACE && T.plon) ts.pl += L.n * step;
-                    if (METHOD == XO_METHOD_MBL) mbl_absorb(L, step);
-                    pend = kEvInteraction;
+                    if (TRACE && T.plon) ts.pl += sl[layer].n * step;
+                    if (METHOD == XO_METHOD_MBL) mbl_absorb(sl[layer], step);
                 }
             }
-            if (alive && pend == kEvInteraction) {
-                /* (C) */
-                const LayerL &L = sl[layer];
-                bool done = false;
-                if (METHOD == XO_METHOD_AR && rng_next(x, a) < lt.w) {
-                    /* albedo rejection: the whole weight is absorbed here,
-                     * mcml.template.c:696-708 */
-                    const float deposit = w;
-                    w -= deposit;
-                    if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
-                    if (use_fluence && deposit_fluence(px, py, pz, deposit, L.mua))
-                        st[XO_STAT_DEPOSITS]++;
-                    done = true;
-                } else {
-                    if (METHOD == XO_METHOD_AW) {
-                        const float deposit = w * lt.w;
-                        w -= deposit;
-                        if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
-                        if (use_fluence && deposit_fluence(px, py, pz, deposit, L.mua))
-                            st[XO_STAT_DEPOSITS]++;
-                    }
-                    float xi_fi;
-                    float ct = pf_sample<PF, true, M>(lpf, lut, x, a, xi_fi);
-                    scatter_direction<M>(dx, dy, dz, ct, xi_fi);
-                    if (TRACE) ts.ev |= XO_EVENT_SCATTERING;
-                    if (METHOD == XO_METHOD_AW && roulette(w, x, a, w_min, chance, use_lottery))
-                        done = true;
-                }
-                end_step(done);
-            }
+            if (inside || (RARE && state == kInteraction)) interact(rare);
+        };
+        /* one round with the rare tests (phase functions whose parameters
+         * the short code does not cover, a degenerate layer's interaction, a
+         * packet near its step limit), or kRoundsPerIteration without: the
+         * loop-top work is shared by that many steps, as in the batch kernel
+         * (1 mm slab 0.464 -> 0.403 ms per 1e6 packets) */
+        if (P.pf_rare || __any(state == kInteraction ||
+                               pkt_steps >= XO_MAX_PACKET_STEPS - kRoundsPerIteration)) {
+            round(std::true_type{});
+        } else {
+#pragma unroll
+            for (uint32_t rep = 0; rep < kRoundsPerIteration; ++rep) round(std::false_type{});
         }
     }
-
+    stat_add(&sstats, XO_STAT_STEPS, pkt_steps);
     if (FLU) cache_flush(fcache, P.accum);
     if (lane_ok) {
         if (!keyed) P.rng_x[gid] = x;
-        if (st[XO_STAT_PACKETS]) st[XO_STAT_THREADS] = 1;
     }
-    stats_flush(&sstats, st, P.stats);
+    stat_add(&sstats, XO_STAT_PACKETS, launched);
+    stat_add(&sstats, XO_STAT_THREADS, launched ? 1u : 0u);
+    stat_add(&sstats, XO_STAT_DEPOSITS, deposits);
+    stats_flush(&sstats, P.stats);
     if (P.lds_bins) {
         for (uint32_t i = tid; i < P.lds_bins; i += blockDim.x)
             if (sbins[i]) atomicAdd(&P.accum[i], sbins[i]);
@@ -577,7 +595,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
     float w = 0.f;
     int32_t vi[3] = {0, 0, 0};
     uint32_t mi = 0;
-    uint32_t st[XO_STAT_COUNT] = {0, 0, 0, 0, 0, 0, 0};
+    uint32_t deposits = 0, launched = 0, steps = 0, faces = 0, crossings = 0;
     uint32_t pkt_steps = 0;
     TraceState ts{0, 0, 0, 0.0f};
     const xo_trace &T = P.trace;
@@ -701,7 +719,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
                                                     : 0u;
             alive = true;
             pkt_steps = 0;
-            st[XO_STAT_PACKETS]++;
+            ++launched;
             if (TRACE) {
                 /* mcvox.template.c:750-756, 1015-1034 */
                 ts = TraceState{pkt_index, 0u, XO_EVENT_LAUNCH, 0.0f};
@@ -742,7 +760,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
             }
             if (!done && ++pkt_steps >= XO_MAX_PACKET_STEPS) {
                 done = true;
-                st[XO_STAT_TRUNCATED]++;
+                stat_add(&sstats, XO_STAT_TRUNCATED, 1u);
             }
             if (TRACE) {
                 /* mcvox.template.c:989-1005 */
@@ -766,7 +784,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
                 w -= deposit;
                 if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
                 if (use_fluence && deposit_fluence(p[0], p[1], p[2], deposit, Mt.mua))
-                    st[XO_STAT_DEPOSITS]++;
+                    ++deposits;
                 done = true;
             } else {
                 if (METHOD == XO_METHOD_AW) {
@@ -775,7 +793,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
                     if (TRACE) ts.ev |= XO_EVENT_ABSORPTION;
                     /* mcsim_fluence_deposit_at, fluence.py:102-147 */
                     if (use_fluence && deposit_fluence(p[0], p[1], p[2], deposit, Mt.mua))
-                        st[XO_STAT_DEPOSITS]++;
+                        ++deposits;
                 }
                 PfL pf{Mt.g, Mt.beta, Mt.la, Mt.lb, Mt.lc, Mt.loff, Mt.lsize_m1};
                 float xi_fi;
@@ -799,7 +817,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
             if (!alive || pend_int) break;
             /* ---- one step of while(!done), mcvox.template.c:748-924 ---- */
             const MaterialL &Mt = sm[mi];
-            st[XO_STAT_STEPS]++;
+            ++steps;
             float step;
             if (METHOD == XO_METHOD_MBL)
                 step = M::div(-M::log_unit(rng_next(x, a)), Mt.mus); /* mcvox.template.c:763-766 */
@@ -837,11 +855,11 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
                             : 0.0f;
                     if (deposit_fluence(p[0] - back * d[0], p[1] - back * d[1],
                                         p[2] - back * d[2], deposit, mua))
-                        st[XO_STAT_DEPOSITS]++;
+                        ++deposits;
                 }
             }
             if (dd < step) {
-                st[XO_STAT_BOUNDARY]++;
+                ++faces;
                 /* mcsim_boundary, mcvox.template.c:275-388 */
                 int32_t nrm[3];
                 nrm[0] = (dist[0] <= dist[1]) && (dist[0] <= dist[2]);
@@ -897,7 +915,7 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
                     vi[1] = nv1;
                     vi[2] = nv2;
                     mi = next_mi;
-                    st[XO_STAT_CROSSINGS]++;
+                    ++crossings;
                     if (escaping) {
                         if (vi[2] < 0)
                             detector_deposit<M>(lds_fresh(sev.top), bins, p[0], p[1], d[0], d[1], d[2],
@@ -918,9 +936,14 @@ __global__ void __launch_bounds__(XO_MAX_BLOCK) mcvox_kernel(const McvoxParams P
     cache_flush(fcache, P.accum);
     if (lane_ok) {
         if (!keyed) P.rng_x[gid] = x;
-        if (st[XO_STAT_PACKETS]) st[XO_STAT_THREADS] = 1;
     }
-    stats_flush(&sstats, st, P.stats);
+    stat_add(&sstats, XO_STAT_PACKETS, launched);
+    stat_add(&sstats, XO_STAT_THREADS, launched ? 1u : 0u);
+    stat_add(&sstats, XO_STAT_STEPS, steps);
+    stat_add(&sstats, XO_STAT_BOUNDARY, faces);
+    stat_add(&sstats, XO_STAT_CROSSINGS, crossings);
+    stat_add(&sstats, XO_STAT_DEPOSITS, deposits);
+    stats_flush(&sstats, P.stats);
     if (P.lds_bins) {
         for (uint32_t i = tid; i < P.lds_bins; i += blockDim.x)
             if (sbins[i]) atomicAdd(&P.accum[i], sbins[i]);

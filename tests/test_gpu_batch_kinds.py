@@ -6,6 +6,7 @@ finite radii must hold the oracle's integers, alone and mixed."""
 import numpy as np
 import pytest
 
+from pyxopto_amd import _native as N
 from pyxopto_amd.mcml import batch as mbatch
 from pyxopto_amd.mcml import mc
 from pyxopto_amd.mcbase import pf as hostpf
@@ -59,3 +60,22 @@ def test_kinds_match_the_oracle(method, rmax):
             lo, n = arr[i].accum_base, arr[i].accum_count
             np.testing.assert_array_equal(acc[lo:lo + n], ref[lo:lo + n],
                                           err_msg=name)
+
+
+@pytest.mark.parametrize('name', list(PFS))
+@pytest.mark.parametrize('method', [0, 1, 2])
+def test_layered_kernel_matches_the_oracle(name, method):
+    print('case', name, method, flush=True)
+    inst = _instance(name, 0, 1.5e-3)
+    sim = mc.Mc(inst.layers, inst.source, inst.detectors,
+                options=[mc.mcoptions.McMethod(method)], rnginit=XINIT)
+    sim.rmax = inst.rmax
+    cfg, lut, naccum = sim.pack()
+    cfg.packet_seed, cfg.first_packet = 0x1234567, 0
+    x, a = N.init_rng(64, XINIT)
+    ref = O.mcml_run(cfg, lut, x, a, 3000, naccum, O.MATH_KERNEL,
+                     keyed=True)[0]
+    for lanes in (64, 0):
+        acc, _ = sim.context.run_mcml(cfg, lut, 3000, naccum, lanes,
+                                      N.XO_FLAG_PACKET_KEYED)
+        np.testing.assert_array_equal(acc, ref)
