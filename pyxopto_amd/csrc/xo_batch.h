@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
 #include <cstring>
 
 #include "../../include/xomc.h"
@@ -37,6 +38,32 @@ struct BatchHdr {
  * step (phase-function kind, source kind, number of layers). */
 inline int item_class(const xo_batch_instance &I) {
     return (I.pf_kind * 4 + I.source_kind) * 16 + (int)I.num_layers;
+}
+
+/* Host: about how many steps the longest packets of an instance take: until
+ * absorption has ended them (the roulette at w_min, or albedo rejection's
+ * one absorption) or they have diffused out of the layers, e-folding in 3 /
+ * pi^2 of the product of the scattering and the transport thickness. A
+ * lookup table counts as g = 0.8. Only its order of magnitude matters. */
+inline double longest_packet(const xo_batch_instance &I, int method, float w_min) {
+    double absorbed = 0.0, scat = 0.0, transport = 0.0;
+    for (uint32_t l = 1; l + 1 < I.num_layers; ++l) {
+        const xo_layer &L = I.layers[l];
+        const double mua = L.mua, mus = L.mus, d = (double)L.bottom - (double)L.top;
+        const double g = I.pf_kind == XO_PF_LUT   ? 0.8
+                         : I.pf_kind == XO_PF_MHG ? (double)L.pf.g * L.pf.beta
+                                                  : (double)L.pf.g;
+        const double folds = method == XO_METHOD_AR ? 10.0 : -std::log((double)w_min + 1e-30);
+        const double n = folds * (1.0 + mus / (mua > 1e-30 ? mua : 1e-30));
+        absorbed = n > absorbed ? n : absorbed;
+        if (mus > 0.0 && d > 0.0) {
+            scat += mus * d;
+            transport += mus * (1.0 - g) * d;
+        }
+    }
+    const double escaped = 10.0 * 0.3 * (scat + 5.0) * (transport + 1.4);
+    const double n = escaped < absorbed ? escaped : absorbed;
+    return n < 1e30 ? n : 1e30; /* also for not a number */
 }
 
 /* Host: the per-instance header of a batch instance; accum_shift is added
@@ -76,6 +103,9 @@ inline bool any_fluence(const BatchHdr *hdr, size_t n) {
         if (hdr[i].fluence.enabled != XO_FLUENCE_NONE) return true;
     return false;
 }
+
+/* Items a wave of the resident grid should find in the queue at least. */
+constexpr uint64_t kItemsPerWave = 2;
 
 /* One work-queue item: packets [first, first + count) of one instance. */
 struct BatchItem {

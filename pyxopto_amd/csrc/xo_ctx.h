@@ -79,16 +79,18 @@ void fill_report(xo_run_report *r, const unsigned long long *stats, uint32_t lan
 
 /* Validate a batch (fn names the entry point in messages) and build its
  * device tables: layer records [instance][XO_BATCH_MAX_LAYERS], per-instance
- * headers and the work items (chunks of opts->chunk packets, grouped by
- * instance class). *total: packets of all instances; *block: threads per
- * block. Returns -1 (message set) on error. */
-int pack_batch(const char *fn, const xo_batch_instance *inst, uint32_t ninst, bool have_lut,
+ * headers and the work items (chunks of at most opts->chunk packets, smaller
+ * ones if `waves` resident waves would find too few; 0: opts->chunk).
+ * *total: packets of all instances; *block: threads per block. Returns -1
+ * (message set) on error. */
+int pack_batch(const char *fn, uint32_t waves, const xo_batch_instance *inst, uint32_t ninst, bool have_lut,
                uint32_t nlut, const xo_batch_opts *opts, uint64_t naccum,
                std::vector<LayerL> &layers, std::vector<BatchHdr> &hdr,
                std::vector<BatchItem> &items, uint64_t *total, uint32_t *block);
 /* The launch options of a batch as kernel parameters (buffers left null). */
 void batch_params(const xo_batch_opts &opts, BatchParams &P);
 /* Blocks of the persistent batch grid for this block size and options. */
+uint32_t batch_waves(xo_ctx *ctx);
 int batch_grid(xo_ctx *ctx, uint32_t block, const xo_batch_opts &opts, uint32_t *blocks);
 
 /* Device layout of a voxel grid: uint8 material indices in 4x4x4 bricks of

@@ -107,7 +107,8 @@ int xo_batch_run_noalloc(xo_ctx *ctx, const xo_batch_instance *inst, uint32_t ni
     std::vector<xo::BatchItem> items;
     uint64_t total = 0;
     uint32_t block = 0;
-    if (xo::pack_batch("xo_batch_run_noalloc", inst, ninst, lut_dev != nullptr, nlut, opts,
+    /* chunks as given: the items have to fit the static array */
+    if (xo::pack_batch("xo_batch_run_noalloc", 0u, inst, ninst, lut_dev != nullptr, nlut, opts,
                        naccum, layers, hdr, items, &total, &block))
         return -1;
     const size_t lbytes = layers.size() * sizeof(xo::LayerL);

@@ -124,8 +124,9 @@ xo_batch_plan *xo_batch_plan_create(xo_ctx *ctx, const xo_batch_instance *inst,
     xo_batch_plan *p = new xo_batch_plan();
     p->ctx = ctx;
     p->naccum = naccum;
-    if (xo::pack_batch("xo_batch_plan_create", inst, ninst, lut != nullptr, nlut, opts, naccum,
-                       layers, hdr, items, &p->total, &p->block)) {
+    if (xo::pack_batch("xo_batch_plan_create", xo::batch_waves(ctx), inst, ninst,
+                       lut != nullptr, nlut, opts, naccum, layers, hdr, items, &p->total,
+                       &p->block)) {
         delete p;
         return nullptr;
     }
