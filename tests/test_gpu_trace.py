@@ -118,6 +118,44 @@ def test_sampling_volume_bit_exact(end_field):
     ctx.close()
 
 
+# packets and events of a row: one packet, rows longer than what a wave stages
+# at a time (256 events, fewer with more packets), one packet more than the
+# waves hold at one and two each, and more than all lanes hold at once
+@pytest.mark.parametrize('npk,maxlen', [(1, 1), (3, 700), (2049, 40),
+                                        (4097, 130), (140001, 9),
+                                        (270000, 3)])
+def test_sampling_volume_shapes_bit_exact(npk, maxlen):
+    print('case', npk, maxlen, flush=True)
+    rng = np.random.default_rng(npk)
+    data = np.zeros((npk, maxlen, N.XO_TRACE_ENTRY_LEN), np.float32)
+    p = rng.uniform(-2e-4, 1.2e-3, (npk, 1, 3)) + \
+        np.cumsum(rng.normal(0, 1e-4, (npk, maxlen, 3)), axis=1)
+    d = np.zeros_like(p)
+    d[:, :-1] = np.diff(p, axis=1)
+    d /= np.maximum(np.linalg.norm(d, axis=2, keepdims=True), 1e-30)
+    data[..., 0:3], data[..., 3:6] = p, d
+    data[..., 6:8] = rng.uniform(0, 1, (npk, maxlen, 2))
+    # axis-parallel and nearly axis-parallel directions, points on faces
+    kind = rng.integers(0, 8, (npk, maxlen))
+    data[..., 3:6][kind == 0] = (0.0, 0.0, 1.0)
+    data[..., 3:6][kind == 1] = (-1.0, 1e-25, -0.0)
+    data[..., 0:3][kind == 2] = np.float32(3e-4)
+    n = rng.integers(0, maxlen + 3, npk).astype(np.int32)
+    n[rng.random(npk) < 0.05] = -1
+    n[-1] = maxlen
+    sv = N.XoSamplingVolume()
+    for i in range(3):
+        sv.top_left[i], sv.voxel_size[i], sv.shape[i] = 0.0, 1e-4, 9 + i
+    sv.multiplier, sv.k, sv.end_field, sv.offset = 1e4, N.XO_ACCU_K, 6, 5
+    ctx = N.Context(0, 0, XINIT)
+    acc, total, rep = ctx.sampling_volume(sv, data, n, 9 * 10 * 11 + 7)
+    racc, rtotal, rcounts = O.sampling_volume(sv, data, n, 9 * 10 * 11 + 7)
+    ctx.close()
+    assert total == rtotal and int(rep.packets) == npk
+    assert [int(rep.steps), int(rep.truncated)] == [int(c) for c in rcounts]
+    np.testing.assert_array_equal(acc, racc)
+
+
 def test_mc_trace_filter_and_sampling_volume():
     T, F = mc.mctrace.Trace, mc.mctrace.Filter
     # packets that leave through the top within 0.5 mm of the source
