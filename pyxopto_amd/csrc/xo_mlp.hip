@@ -284,6 +284,83 @@ mlp_fused_kernel(const FusedArgs f) {
     fused_layer<8, 2, true>(f, f.nlayers - 1, hb, row0, lane, wave);
 }
 
+/* The same products for few rows. With at most one block per CU, the time is
+ * that of one block: of the weights' way from L2 (270 KB for 256-wide hidden
+ * layers, 64 bytes per clock and CU at best). A block of 16 waves takes 16
+ * rows, each wave one 16-column tile, and every wave requests a layer's whole
+ * weights while the layer before is computed: they do not depend on the
+ * rows. The k order of each result is that of mlp_fused_kernel, and so are
+ * its bits. 64 rows 13.0 -> 8.1 us (mostly the launch), 4096 rows 16.9 ->
+ * 10.1. */
+constexpr int SWAVES = 16, SROWS = 16;
+
+/* Fragments of wave's tile of hidden or last layer l >= 1. */
+__device__ __forceinline__ void small_weights(const FusedArgs &f, int l, int lane, int wave,
+                                              bf16x8 b[8]) {
+    if (l + 1 == f.nlayers && wave >= 8) return; /* the last layer has 8 tiles */
+    const uint16_t *wp = f.wt[l] + ((size_t)wave * 8 * 64 + lane) * 8;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) b[s] = *reinterpret_cast<const bf16x8 *>(wp + s * 512);
+}
+
+__global__ void __launch_bounds__(64 * SWAVES) mlp_fused_small_kernel(const FusedArgs f) {
+    __shared__ __attribute__((aligned(16))) uint16_t hb[2][SROWS * FSTRIDE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int fr = lane & 15, fk = (lane >> 4) * 8, nq = (lane >> 4) * 4;
+    const int row0 = blockIdx.x * SROWS;
+    const int m0 = tid >> 5, c0 = tid & 31;
+    float xv = 0.f;
+    if (tid < 32 * SROWS && row0 + m0 < f.M && c0 < f.nin)
+        xv = f.X[(size_t)(row0 + m0) * f.nin + c0];
+    const bf16x8 first =
+        *reinterpret_cast<const bf16x8 *>(f.wt[0] + ((size_t)wave * 64 + lane) * 8);
+    bf16x8 b[8], next[8];
+    small_weights(f, 1, lane, wave, b);
+    if (tid < 32 * SROWS) hb[0][m0 * FSTRIDE + c0] = f2bf(xv);
+    __syncthreads();
+    for (int l = 0; l < f.nlayers; ++l) {
+        const bool last = l + 1 == f.nlayers;
+        const uint16_t *in = &hb[l & 1][fr * FSTRIDE + fk];
+        floatx4 acc = floatx4{0.f, 0.f, 0.f, 0.f};
+        if (l == 0) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                first, *reinterpret_cast<const bf16x8 *>(in), acc, 0, 0, 0);
+        } else {
+            if (!last) small_weights(f, l + 1, lane, wave, next);
+            if (last && wave >= 8) return;
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    b[s], *reinterpret_cast<const bf16x8 *>(in + s * 32), acc, 0, 0, 0);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) b[s] = next[s];
+        }
+        const float *bias = f.bias[l];
+        const int n0 = wave * 16 + nq;
+        if (!last) {
+            const float4 bv = *reinterpret_cast<const float4 *>(bias + n0);
+            const float z0 = acc[0] + bv.x, z1 = acc[1] + bv.y;
+            const float z2 = acc[2] + bv.z, z3 = acc[3] + bv.w;
+            uint2 pk;
+            pk.x = bf16_pair(z0 > 0.f ? z0 : 0.f, z1 > 0.f ? z1 : 0.f);
+            pk.y = bf16_pair(z2 > 0.f ? z2 : 0.f, z3 > 0.f ? z3 : 0.f);
+            *reinterpret_cast<uint2 *>(&hb[(l + 1) & 1][fr * FSTRIDE + n0]) = pk;
+            __syncthreads(); /* the other tile holds this layer's output */
+        } else if (row0 + fr < f.M && n0 < f.nout) {
+            float *y = f.Y + (size_t)(row0 + fr) * f.nout + n0;
+            if ((f.nout & 3) == 0) { /* n0 + 3 < nout, 16-byte aligned */
+                *reinterpret_cast<float4 *>(y) =
+                    make_float4(acc[0] + bias[n0], acc[1] + bias[n0 + 1], acc[2] + bias[n0 + 2],
+                                acc[3] + bias[n0 + 3]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (n0 + q < f.nout) y[q] = acc[q] + bias[n0 + q];
+            }
+        }
+    }
+}
+
 /* A matrix M[k][n] (k < kdim, n < ndim) as bf16 MFMA fragments: for
  * 16-column tile t, 32-wide k step s and lane L, the 8 values M[k][n] with
  * n = 16 t + (L & 15), k = 32 s + 8 (L >> 4) + e (e = 0..7) are stored at
@@ -1270,6 +1347,12 @@ __global__ void __launch_bounds__(WNT) train_weights_kernel(const WgArgs g) {
 
 } // namespace
 
+/* A forward pass whose rows and outputs fit is read and written by the kernel
+ * in pinned memory: no copy to queue on either side (64 rows 46 -> 23.5 us,
+ * 2480 rows 82 -> 65, 4096 rows 129 -> 109). The gain shrinks with the copy
+ * out of it: 5 % at 9900 rows. */
+constexpr uint64_t kStageBytes = 2048u * 1024u;
+
 struct xo_mlp {
     xo_ctx *ctx = nullptr;
     hipStream_t stream = nullptr;
@@ -1304,6 +1387,9 @@ struct xo_mlp {
     uint16_t *zrow = nullptr;         /* zeros read for rows past a layer's width */
     float *loss_part = nullptr;       /* fused step: one partial loss per row block */
     bool fusable = false, train_fused = false, wt_dirty = true;
+    float *stage = nullptr;           /* kStageBytes of pinned memory: the rows of a small
+                                         forward pass, then their outputs */
+    hipEvent_t ev0 = nullptr, ev1 = nullptr; /* around a forward pass's kernels */
     float *loss = nullptr;            /* per training step */
     uint32_t loss_cap = 0;
     uint32_t *step = nullptr;         /* [0] the step counter, [1] the fused step's copy */
@@ -1612,12 +1698,12 @@ int train_fused_step(xo_mlp *N, uint32_t B, const float *X, const LossSpec &loss
     return 0;
 }
 
-/* Fused forward pass of B rows in N->xf (fp32) into N->y. */
-int forward_fused(xo_mlp *N, uint32_t B) {
+/* Fused forward pass of the B rows x (fp32) into y, device or pinned memory. */
+int forward_fused(xo_mlp *N, uint32_t B, const float *x, float *y) {
     FusedArgs f;
     std::memset(&f, 0, sizeof(f));
-    f.X = N->xf;
-    f.Y = N->y;
+    f.X = x;
+    f.Y = y;
     f.M = (int)B;
     f.nin = N->dims[0];
     f.nout = N->dims[N->nlayers];
@@ -1626,7 +1712,15 @@ int forward_fused(xo_mlp *N, uint32_t B) {
         f.wt[l] = N->wt + N->wt_off[l];
         f.bias[l] = N->w + N->boff[l];
     }
-    hipLaunchKernelGGL(mlp_fused_kernel, dim3((B + FBM - 1) / FBM), dim3(256), 0, N->stream, f);
+    /* one block per CU at most (4096 rows 16.9 -> 10.1 us); with more, the
+     * weights would pass each CU again for every 16 rows instead of 64 */
+    const uint32_t small = (B + SROWS - 1) / SROWS;
+    if (small <= N->ctx->cus)
+        hipLaunchKernelGGL(mlp_fused_small_kernel, dim3(small), dim3(64 * SWAVES), 0, N->stream,
+                           f);
+    else
+        hipLaunchKernelGGL(mlp_fused_kernel, dim3((B + FBM - 1) / FBM), dim3(256), 0, N->stream,
+                           f);
     MLP_CHECK(hipGetLastError());
     return 0;
 }
@@ -1702,6 +1796,9 @@ void xo_mlp_destroy(xo_mlp *N) {
             if (p) (void)hipFree(p);
     for (auto &kv : N->dw_tables)
         if (kv.second) (void)hipFree(kv.second);
+    if (N->stage) (void)hipHostFree(N->stage);
+    if (N->ev0) (void)hipEventDestroy(N->ev0);
+    if (N->ev1) (void)hipEventDestroy(N->ev1);
     if (N->stream) (void)hipStreamDestroy(N->stream);
     delete N;
 }
@@ -1879,34 +1976,47 @@ int xo_mlp_forward(xo_mlp *N, const float *x, uint64_t n, float *y, double *kern
     std::lock_guard<std::mutex> lock(N->mu);
     MLP_CHECK(hipSetDevice(N->ctx->device));
     const uint32_t nin = N->dims[0], nout = N->dims[N->nlayers];
-    hipEvent_t e0, e1;
-    MLP_CHECK(hipEventCreate(&e0));
-    MLP_CHECK(hipEventCreate(&e1));
+    if (!N->ev0) MLP_CHECK(hipEventCreate(&N->ev0));
+    if (!N->ev1) MLP_CHECK(hipEventCreate(&N->ev1));
+    if (N->fusable && !N->stage &&
+        hipHostMalloc((void **)&N->stage, kStageBytes, hipHostMallocDefault) != hipSuccess) {
+        N->stage = nullptr; /* copies then */
+        (void)hipGetLastError();
+    }
     double total = 0.0;
     int rc = 0;
     if (N->fusable && N->wt_dirty && refresh_transposed(N)) rc = -1;
     for (uint64_t r = 0; r < n && rc == 0; r += N->max_batch) {
         const uint32_t B = (uint32_t)(n - r < N->max_batch ? n - r : N->max_batch);
-        if (N->fusable) {
-            if (hipMemcpyAsync(N->xf, x + r * nin, sizeof(float) * B * nin,
-                               hipMemcpyHostToDevice, N->stream) != hipSuccess) { rc = -1; break; }
+        const uint64_t xbytes = 4ull * B * nin, ybytes = 4ull * B * nout;
+        /* the outputs start on a 16-byte boundary, as in N->y */
+        const uint64_t ystart = (xbytes + 15u) & ~(uint64_t)15u;
+        const bool staged = N->stage && ystart + ybytes <= kStageBytes;
+        float *ys = staged ? N->stage + ystart / 4u : N->y;
+        if (staged) {
+            std::memcpy(N->stage, x + r * nin, xbytes);
+        } else if (N->fusable) {
+            if (hipMemcpyAsync(N->xf, x + r * nin, xbytes, hipMemcpyHostToDevice, N->stream) !=
+                hipSuccess) { rc = -1; break; }
         } else if (upload_rows(N, x + r * nin, B)) { rc = -1; break; }
-        if (hipEventRecord(e0, N->stream) != hipSuccess) { rc = -1; break; }
-        if (N->fusable ? forward_fused(N, B) : forward(N, B)) { rc = -1; break; }
-        if (hipEventRecord(e1, N->stream) != hipSuccess) { rc = -1; break; }
-        if (hipMemcpyAsync(y + r * nout, N->y, 4ull * B * nout, hipMemcpyDeviceToHost,
-                           N->stream) != hipSuccess ||
+        if (hipEventRecord(N->ev0, N->stream) != hipSuccess) { rc = -1; break; }
+        if (N->fusable ? forward_fused(N, B, staged ? N->stage : N->xf, ys) : forward(N, B)) {
+            rc = -1;
+            break;
+        }
+        if (hipEventRecord(N->ev1, N->stream) != hipSuccess) { rc = -1; break; }
+        if ((!staged && hipMemcpyAsync(y + r * nout, N->y, ybytes, hipMemcpyDeviceToHost,
+                                       N->stream) != hipSuccess) ||
             hipStreamSynchronize(N->stream) != hipSuccess) {
             xo::set_error("xo_mlp_forward: device failure");
             rc = -1;
             break;
         }
+        if (staged) std::memcpy(y + r * nout, ys, ybytes);
         float ms = 0.f;
-        (void)hipEventElapsedTime(&ms, e0, e1);
+        (void)hipEventElapsedTime(&ms, N->ev0, N->ev1);
         total += ms;
     }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
     if (kernel_ms) *kernel_ms = total;
     return rc;
 }

@@ -132,6 +132,33 @@ def test_fused_inference_equals_layer_by_layer(ctx, rows):
     net.close()
 
 
+@pytest.mark.parametrize('dims', [S.DIMS, (1, 256, 1), (32, 256, 256, 127),
+                                  (7,) + (256,) * 7 + (128,)])
+def test_forward_of_few_rows_equals_forward_of_many(ctx, dims):
+    """Up to 16 rows per CU run in 16-row blocks, more in 64-row blocks, and
+    what fits 2 MiB is passed in pinned memory: the same products in the
+    same order, so a row's outputs are the same bits in every call."""
+    net = S.Network(dims, ctx, max_batch=9000)
+    rng = np.random.default_rng(len(dims))
+    p = M.init_params(dims, seed=3)
+    p += rng.normal(0, 0.02, p.size).astype(np.float32)
+    net.set_params(p)
+    x = rng.uniform(-1, 1, (9000, dims[0])).astype(np.float32)
+    y, _ = net.forward(x)
+    yref, _ = M.forward(p, x[:500], dims, emulate_bf16=True)
+    # the bound of the flips of bf16 roundings above, per layer of S.DIMS
+    assert np.linalg.norm(y[:500] - yref) / np.linalg.norm(yref) < \
+        1e-3 * max(1.0, len(dims) / len(S.DIMS))
+    fit = 2 ** 21 // (4 * (dims[0] + dims[-1]))
+    for rows in {1, 15, 16, 17, 100, min(fit - 4, 9000), min(fit + 4, 9000),
+                 4095, 4096, 4097}:
+        print('case', dims, rows, flush=True)
+        lo = int(rng.integers(0, 9000 - rows + 1))
+        ys, _ = net.forward(x[lo:lo + rows])
+        np.testing.assert_array_equal(ys, y[lo:lo + rows])
+    net.close()
+
+
 @pytest.mark.parametrize('dims', [(5, 64, 64, 10), S.DIMS, (5, 256, 100),
                                   (5, 256, 256, 256, 256, 256, 128)])
 def test_captured_steps_equal_eager_steps(ctx, dims):
