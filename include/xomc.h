@@ -132,7 +132,10 @@ enum xo_run_flags {
      * reference makes with -cl-fast-relaxed-math (xopto/cl/cloptions.py:
      * 137-152; test/performance.py:104). Results then agree with the exact
      * build statistically, not bit for bit. Ignored by traced runs. */
-    XO_FLAG_FAST_MATH = 1u << 3
+    XO_FLAG_FAST_MATH = 1u << 3,
+    /* The caller's trace_data is all zeros: the entries past a packet's last
+     * event are then left as they are instead of being written. */
+    XO_FLAG_TRACE_ZEROED = 1u << 4
 };
 
 /* Phase-function parameters; the union of McPf for Hg, MHg and Lut. */
@@ -363,7 +366,9 @@ typedef struct xo_batch_instance {
 
 /* Launch shape of a batch run (chosen by the autotuner). */
 typedef struct xo_batch_opts {
-    uint32_t chunk;             /* packets per work-queue item (>= 1)        */
+    uint32_t chunk;             /* packets per work-queue item (>= 1), at most:
+                                   fewer where a launch would otherwise leave
+                                   waves without items                        */
     uint32_t block;             /* threads per block: 64, 128 or 256          */
     uint32_t blocks_per_cu;     /* 0: as many as fit                          */
     uint32_t flags;             /* XO_FLAG_FAST_MATH; other flags are ignored */
@@ -373,7 +378,8 @@ typedef struct xo_batch_opts {
     uint32_t refill_min;        /* a wave hands out new packets once this
                                    many of its lanes are idle (0: 4)          */
     uint32_t defer_min;         /* a wave handles its boundary events once
-                                   this many lanes hold one (0: 16)           */
+                                   this many of 64 live lanes hold one
+                                   (0: 16)                                    */
     int32_t method;             /* enum xo_method of every instance           */
 } xo_batch_opts;
 
@@ -462,7 +468,8 @@ int xo_mcml_run(xo_ctx *ctx, const xo_mcml_cfg *cfg,
  * McKernel, xopto/mcml/kernel/mcml.template.c:513-520, 764-810, and
  * mcsim_trace_event / mcsim_trace_complete of xopto/mcbase/mctrace.py:
  * 519-566). trace_data: host output of npackets * max_events *
- * XO_TRACE_ENTRY_LEN floats; trace_n: host output of npackets event counts.
+ * XO_TRACE_ENTRY_LEN floats (entries past a packet's last event: 0);
+ * trace_n: host output of npackets event counts.
  * Row p holds packet p (the packet index of the run). */
 int xo_mcml_run_trace(xo_ctx *ctx, const xo_mcml_cfg *cfg,
                       const float *lut, uint32_t nlut,

@@ -44,6 +44,7 @@ XO_FLAG_STATIC_SCHEDULE = 1 << 0
 XO_FLAG_NO_LDS_BINS = 1 << 1
 XO_FLAG_PACKET_KEYED = 1 << 2
 XO_FLAG_FAST_MATH = 1 << 3
+XO_FLAG_TRACE_ZEROED = 1 << 4
 (XO_MATH_LOG, XO_MATH_SIN_TURNS, XO_MATH_COS_TURNS, XO_MATH_SQRT, XO_MATH_RCP,
  XO_MATH_RSQRT, XO_MATH_CBRT, XO_MATH_EXP) = range(8)
 
@@ -578,7 +579,8 @@ class Context:
         rep = XoRunReport()
         check(lib().xo_mcml_run_trace(
             self._h, ctypes.byref(cfg), lut_p, c_uint32(nlut),
-            c_uint64(npackets), c_uint32(lanes), c_uint32(flags),
+            c_uint64(npackets), c_uint32(lanes),
+            c_uint32(flags | XO_FLAG_TRACE_ZEROED),
             ctypes.byref(trace), _ptr(data, c_float), _ptr(n, c_int32),
             _ptr(accum, c_uint64), c_uint64(naccum), ctypes.byref(rep)),
             'xo_mcml_run_trace')
@@ -716,7 +718,8 @@ class Context:
             check(lib().xo_mcvox_run_trace(
                 self._h, ctypes.byref(cfg), vox_p, c_uint64(nvox), lut_p,
                 c_uint32(nlut), c_uint64(npackets), c_uint32(lanes),
-                c_uint32(flags), ctypes.byref(trace), _ptr(data, c_float),
+                c_uint32(flags | XO_FLAG_TRACE_ZEROED), ctypes.byref(trace),
+                _ptr(data, c_float),
                 _ptr(n, c_int32), _ptr(accum, c_uint64), c_uint64(naccum),
                 ctypes.byref(rep)), 'xo_mcvox_run_trace')
             return accum, rep, data, n

@@ -622,6 +622,7 @@ void xo_ctx_destroy(xo_ctx *ctx) {
     if (ctx->batch_items) (void)hipFree(ctx->batch_items);
     if (ctx->trace_data) (void)hipFree(ctx->trace_data);
     if (ctx->trace_n) (void)hipFree(ctx->trace_n);
+    if (ctx->trace_stage) (void)hipHostFree(ctx->trace_stage);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
@@ -717,12 +718,87 @@ static int trace_buffers(xo_ctx *ctx, uint64_t floats, uint64_t npackets) {
     return 0;
 }
 
+/* Pinned memory that a trace passes through, and the packets of one pass: the
+ * used entries, then the first entry of each packet. */
+constexpr uint64_t kTraceStage = 4u << 20;
+constexpr uint32_t kTracePackets = 65536;
+/* Traces of less are copied whole (a megabyte takes less than the launch and
+ * the wait of a pass). */
+constexpr uint64_t kTraceWhole = 1u << 20;
+
+/* One wave copies the used entries of a packet to their place in the pass: a
+ * row holds max_events entries, of which packets use a tenth or so, and the
+ * way to the host is what bounds it. */
+static __global__ void __launch_bounds__(256)
+pack_trace_kernel(const float4 *data, const int32_t *n, uint32_t max_events, uint32_t count,
+                  const uint32_t *first, float4 *out) {
+    const uint32_t p = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (p >= count) return;
+    const int32_t c = n[p];
+    const uint32_t used = c <= 0 ? 0u : ((uint32_t)c < max_events ? (uint32_t)c : max_events);
+    const float4 *src = data + (uint64_t)p * max_events * (XO_TRACE_ENTRY_LEN / 4);
+    float4 *dst = out + (uint64_t)first[p] * (XO_TRACE_ENTRY_LEN / 4);
+    for (uint32_t i = threadIdx.x & 63u; i < used * (XO_TRACE_ENTRY_LEN / 4); i += 64u)
+        dst[i] = src[i];
+}
+
+/* The trace into the caller's buffers. zeroed: the caller's data is all
+ * zeros, so only the used entries are brought over (5000 packets of 300
+ * entries, 12 % used: run 5.5 -> 2.7 ms), unless most
+ * are used. */
 static int trace_download(xo_ctx *ctx, float *data, int32_t *n, uint64_t floats,
-                          uint64_t npackets) {
+                          uint64_t npackets, const xo_trace &trace, bool zeroed) {
     if (!npackets) return 0;
-    XO_HIP(hipMemcpyAsync(data, ctx->trace_data, floats * 4, hipMemcpyDeviceToHost,
-                          ctx->stream));
     XO_HIP(hipMemcpyAsync(n, ctx->trace_n, npackets * 4, hipMemcpyDeviceToHost, ctx->stream));
+    const uint64_t row = (uint64_t)trace.max_events * XO_TRACE_ENTRY_LEN;
+    bool packed = zeroed && floats * 4 > kTraceWhole && row * 4 <= kTraceStage;
+    if (packed && !ctx->trace_stage &&
+        hipHostMalloc((void **)&ctx->trace_stage, kTraceStage + 4u * kTracePackets,
+                      hipHostMallocDefault) != hipSuccess) {
+        ctx->trace_stage = nullptr;
+        (void)hipGetLastError();
+        packed = false;
+    }
+    auto used = [&](uint64_t p) {
+        return (uint64_t)std::min(std::max(n[p], 0), trace.max_events);
+    };
+    if (packed) {
+        XO_HIP(hipStreamSynchronize(ctx->stream));
+        uint64_t entries = 0;
+        for (uint64_t p = 0; p < npackets; ++p) entries += used(p);
+        packed = 2u * entries <= npackets * (uint64_t)trace.max_events;
+    }
+    if (!packed) {
+        XO_HIP(hipMemcpyAsync(data, ctx->trace_data, floats * 4, hipMemcpyDeviceToHost,
+                              ctx->stream));
+        return 0;
+    }
+    const uint64_t entry = 4u * XO_TRACE_ENTRY_LEN; /* bytes */
+    float *stage = ctx->trace_stage;
+    uint32_t *first = reinterpret_cast<uint32_t *>((char *)stage + kTraceStage);
+    for (uint64_t p0 = 0; p0 < npackets;) {
+        uint32_t count = 0;
+        uint64_t filled = 0;
+        while (p0 + count < npackets && count < kTracePackets &&
+               (filled + used(p0 + count)) * entry <= kTraceStage) {
+            first[count] = (uint32_t)filled;
+            filled += used(p0 + count);
+            ++count;
+        }
+        if (filled) {
+            hipLaunchKernelGGL(pack_trace_kernel, dim3((count + 3u) / 4u), dim3(256), 0,
+                               ctx->stream,
+                               reinterpret_cast<const float4 *>(ctx->trace_data + p0 * row),
+                               ctx->trace_n + p0, (uint32_t)trace.max_events, count, first,
+                               reinterpret_cast<float4 *>(stage));
+            XO_HIP(hipGetLastError());
+            XO_HIP(hipStreamSynchronize(ctx->stream));
+            for (uint32_t k = 0; k < count; ++k)
+                std::memcpy(data + (p0 + k) * row, (const char *)stage + first[k] * entry,
+                            used(p0 + k) * entry);
+        }
+        p0 += count;
+    }
     return 0;
 }
 
@@ -838,7 +914,9 @@ static int mcml_run(xo_ctx *ctx, const xo_mcml_cfg *cfg, const float *lut, uint3
     XO_HIP(hipEventRecord(ctx->ev1, ctx->stream));
     unsigned long long stats[1 + XO_STAT_COUNT];
     XO_HIP(hipMemcpyAsync(accum, ctx->accum, naccum * 8, hipMemcpyDeviceToHost, ctx->stream));
-    if (trace && trace_download(ctx, trace_data, trace_n, trace_floats, npackets)) return -1;
+    if (trace && trace_download(ctx, trace_data, trace_n, trace_floats, npackets, *trace,
+                                (flags & XO_FLAG_TRACE_ZEROED) != 0u))
+        return -1;
     XO_HIP(hipMemcpyAsync(stats, ctx->counters, sizeof(stats), hipMemcpyDeviceToHost,
                           ctx->stream));
     XO_HIP(hipStreamSynchronize(ctx->stream));
@@ -1012,7 +1090,9 @@ static int mcvox_run(xo_ctx *ctx, const xo_mcvox_cfg *cfg, const int32_t *voxels
     XO_HIP(hipEventRecord(ctx->ev1, ctx->stream));
     unsigned long long stats[1 + XO_STAT_COUNT];
     XO_HIP(hipMemcpyAsync(accum, ctx->accum, naccum * 8, hipMemcpyDeviceToHost, ctx->stream));
-    if (trace && trace_download(ctx, trace_data, trace_n, trace_floats, npackets)) return -1;
+    if (trace && trace_download(ctx, trace_data, trace_n, trace_floats, npackets, *trace,
+                                (flags & XO_FLAG_TRACE_ZEROED) != 0u))
+        return -1;
     XO_HIP(hipMemcpyAsync(stats, ctx->counters, sizeof(stats), hipMemcpyDeviceToHost,
                           ctx->stream));
     XO_HIP(hipStreamSynchronize(ctx->stream));

@@ -59,6 +59,7 @@ struct xo_ctx {
     size_t trace_data_cap = 0;
     int32_t *trace_n = nullptr;
     size_t trace_n_cap = 0;
+    float *trace_stage = nullptr; /* pinned; a trace on its way to the host */
     std::mutex mu;
 };
 

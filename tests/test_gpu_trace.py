@@ -93,6 +93,32 @@ def test_keyed_trace_rows_independent_of_schedule():
     ctx.close()
 
 
+# entries per row and packets: traces passed whole (up to 1 MiB, or mostly
+# used) or their used entries only, in one pass and in several (more than
+# 65536 packets, more than 4 MiB used)
+@pytest.mark.parametrize('npk,maxlen,options', [
+    (4096, 8, N.XO_TRACE_START | N.XO_TRACE_END),
+    (4097, 8, N.XO_TRACE_START | N.XO_TRACE_END),
+    (70000, 8, N.XO_TRACE_START | N.XO_TRACE_END),
+    (70000, 3, N.XO_TRACE_START | N.XO_TRACE_END),
+    (9000, 300, N.XO_TRACE_ALL)])
+def test_trace_transfer_bit_exact(npk, maxlen, options):
+    print('case', npk, maxlen, options, flush=True)
+    cfg, lut, naccum = _sim(0).pack()
+    cfg.packet_seed, cfg.first_packet = 0x5EED, 0
+    trace = _xt(maxlen, options)
+    ctx = N.Context(0, 0, XINIT)
+    acc, rep, data, n = ctx.run_mcml_trace(cfg, lut, npk, naccum, trace, 0,
+                                           N.XO_FLAG_PACKET_KEYED)
+    ctx.close()
+    x, a = N.init_rng(1024, XINIT)
+    racc, _, _, rdata, rn = O.mcml_run_trace(
+        cfg, lut, x, a, npk, naccum, trace, O.MATH_KERNEL, keyed=True)
+    np.testing.assert_array_equal(n, rn)
+    np.testing.assert_array_equal(data, rdata)
+    np.testing.assert_array_equal(acc, racc)
+
+
 @pytest.mark.parametrize('end_field', [6, 7])
 def test_sampling_volume_bit_exact(end_field):
     sim = _sim(0)
