@@ -41,7 +41,8 @@ SERVING_QPS = 250.0                     # requests/s of the serving run
 # 1 GiB device-to-device copy (profiles/batch_kernel_layered_batch_4096.md,
 # profiles/mcvox_kernel_skin_vessel_200.md,
 # profiles/mcml_kernel_slab_1mm_and_surrogate.md). Offline figures: measured
-# for the kernels as they are in this tree, hardware arithmetic.
+# with the builds that those profiles name, hardware arithmetic; a larger fluence
+# window has since taken some of skin_vessel_200's atomics into LDS.
 TRAFFIC_BYTES_PER_LAUNCH = {'layered_batch_4096': 2.585e11,
                             'skin_vessel_200': 7.52e11,
                             'slab_1mm': 5.3e6}
