@@ -109,8 +109,6 @@ struct McvoxParams {
     uint32_t lds_bins;
     uint32_t lds_lut;
     FluenceL fluence;      /* the grid of cfg.fluence, with its window    */
-    uint32_t pf_rare;      /* some medium needs the general phase-function
-                              sampling code (xo::pf_rare)                 */
 };
 
 /* Largest window: zeroing and adding it up costs every block about a

@@ -9,7 +9,8 @@
  * mcml.template.c:460, 790-812); with the static schedule lane g runs packets
  * g, g+L, ... . The layer/material table is staged once per block in LDS;
  * detector bins are privatized in LDS when they fit and flushed with one u64
- * atomic per bin and block; fluence deposits are u64 atomics to HBM.
+ * atomic per bin and block; so is a window of the fluence grid, deposits
+ * outside of it are u64 atomics to HBM.
  * Everything is binary32 VALU work; nothing here is a contraction, so no MFMA.
  */
 #include <hip/hip_runtime.h>
