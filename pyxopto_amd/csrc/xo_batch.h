@@ -19,20 +19,23 @@ namespace xo {
 
 /* Per-instance constants the lanes read at packet launch and escape. */
 struct BatchHdr {
-    int32_t num_layers;
+    uint64_t seed;
+    uint16_t num_layers;
+    uint16_t src_kind;          /* XO_SRC_LINE, _FIBER_NI or _FIBER */
     int32_t pf_kind;
     float rmax2;
     float reflectance;
     float src_pos[3];           /* Line: surface point; fiber: core centre */
     float dir_sample[3];
     float dir_reflected[3];
-    int32_t src_kind;           /* XO_SRC_LINE, _FIBER_NI or _FIBER */
-    uint64_t seed;
     xo_detector top, bottom, specular;
     xo_source_fiber fiber;
     xo_fiber_axis fiber_axis;
-    FluenceL fluence;           /* enabled 0: none */
+    FluenceGrid fluence;        /* enabled 0: none */
 };
+/* XO_NOALLOC_SCRATCH_BYTES holds the headers of a batch: a larger one would
+ * refuse batches that fit. */
+static_assert(sizeof(BatchHdr) <= 344, "batch header grown");
 
 /* Host: instances of one class run the same branches of the transport
  * step (phase-function kind, source kind, number of layers). */
@@ -72,10 +75,10 @@ inline BatchHdr batch_header(const xo_batch_instance &I, const xo_detector det[3
                              uint32_t accum_shift) {
     BatchHdr H;
     std::memset(&H, 0, sizeof(H));
-    H.num_layers = (int32_t)I.num_layers;
+    H.num_layers = (uint16_t)I.num_layers;
     H.pf_kind = I.pf_kind;
     H.rmax2 = I.rmax * I.rmax;
-    H.src_kind = I.source_kind;
+    H.src_kind = (uint16_t)I.source_kind;
     H.fiber = I.fiber;
     H.fiber_axis = I.fiber_axis;
     const bool fiber = I.source_kind == XO_SRC_FIBER_NI || I.source_kind == XO_SRC_FIBER;
@@ -92,7 +95,7 @@ inline BatchHdr batch_header(const xo_batch_instance &I, const xo_detector det[3
     H.top.offset += accum_shift;
     H.bottom.offset += accum_shift;
     H.specular.offset += accum_shift;
-    H.fluence = fluence_to_device(I.fluence);
+    H.fluence = fluence_without_window(fluence_to_device(I.fluence));
     if (H.fluence.enabled != XO_FLUENCE_NONE) H.fluence.offset += accum_shift;
     return H;
 }

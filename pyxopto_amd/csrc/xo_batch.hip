@@ -254,7 +254,7 @@ batch_kernel(const BatchParams P) {
         /* an instance's fluence deposit (fluence.py:102-147); the grid is
          * read from the instance header only when the batch has one */
         auto fluence_at = [&](float qx, float qy, float qz, float deposit, float mua) {
-            const FluenceL &F = P.hdr[inst].fluence;
+            const FluenceGrid &F = P.hdr[inst].fluence;
             if (F.enabled != XO_FLUENCE_NONE &&
                 fluence_deposit<M>(F, P.accum, qx, qy, qz, deposit, mua))
                 count(kCounts - 1, 1u);

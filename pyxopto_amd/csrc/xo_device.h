@@ -305,10 +305,13 @@ XO_DEV void cache_flush(FluenceCache &c, unsigned long long *accum) {
     c.index = 0xFFFFFFFFu;
 }
 
-/* The weight a fluence accumulator adds for an absorbed weight w: w in
+/* Deposits into a fluence grid G (FluenceL or FluenceGrid).
+ *
+ * The weight a fluence accumulator adds for an absorbed weight w: w in
  * deposition mode, w / mua in fluence-rate mode (0 where mua is 0),
  * fluence.py:139-141. */
-template <class M = MathExact> XO_DEV float fluence_weight(const FluenceL &F, float w, float mua) {
+template <class M = MathExact, class G>
+XO_DEV float fluence_weight(const G &F, float w, float mua) {
     if (F.rate) w *= (mua != 0.0f) ? M::div(1.0f, mua) : 0.0f;
     return w;
 }
@@ -316,8 +319,8 @@ template <class M = MathExact> XO_DEV float fluence_weight(const FluenceL &F, fl
 /* Bin (x, y, z) of a point: the Cartesian voxel of mcsim_fluence_deposit_at
  * (fluence.py:102-147) or the (r, 0, z) cell of fluencerz.py:112-160; false
  * outside the grid. */
-template <class M = MathExact>
-XO_DEV bool fluence_bin(const FluenceL &F, float px, float py, float pz, uint32_t &ix,
+template <class M = MathExact, class G>
+XO_DEV bool fluence_bin(const G &F, float px, float py, float pz, uint32_t &ix,
                         uint32_t &iy, uint32_t &iz) {
     const float ddx = px - F.top_left[0];
     const float ddy = py - F.top_left[1];
@@ -346,21 +349,22 @@ XO_DEV bool fluence_bin(const FluenceL &F, float px, float py, float pz, uint32_
 }
 
 /* Accumulator index of a fluence bin: x (or r) fastest. */
-XO_DEV uint64_t fluence_index(const FluenceL &F, uint32_t ix, uint32_t iy, uint32_t iz) {
+template <class G>
+XO_DEV uint64_t fluence_index(const G &F, uint32_t ix, uint32_t iy, uint32_t iz) {
     return F.offset + ((uint64_t)iz * F.ny + iy) * F.nx + ix;
 }
 
 /* Integer weight of a deposit; mua is that of the medium the packet is in
  * (used in fluence-rate mode). */
-template <class M = MathExact>
-XO_DEV uint32_t fluence_integer(const FluenceL &F, float w, float mua) {
+template <class M = MathExact, class G>
+XO_DEV uint32_t fluence_integer(const G &F, float w, float mua) {
     return f2u_sat(fluence_weight<M>(F, w, mua) * F.k + 0.5f);
 }
 
 /* Fluence deposit at a point. Returns true if a non-zero integer was
  * added. */
-template <class M = MathExact>
-XO_DEV bool fluence_deposit(const FluenceL &F, unsigned long long *accum, float px,
+template <class M = MathExact, class G>
+XO_DEV bool fluence_deposit(const G &F, unsigned long long *accum, float px,
                             float py, float pz, float w, float mua) {
     uint32_t ix, iy, iz;
     if (!fluence_bin<M>(F, px, py, pz, ix, iy, iz)) return false;

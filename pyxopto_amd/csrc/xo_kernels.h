@@ -33,7 +33,7 @@ enum {
 
 namespace xo {
 
-/* A fluence grid as the kernels read it per deposit, in five 16-byte words.
+/* A fluence grid as the single-simulation kernels read it per deposit.
  * origin, ext, bins: the box of bins (x or r, y, z; x fastest) that a block
  * of a single-simulation kernel accumulates in LDS and adds to the
  * accumulator once; bins 0: none. */
@@ -66,6 +66,26 @@ inline FluenceL fluence_to_device(const xo_fluence &F) {
     o.ny = F.enabled == XO_FLUENCE_XYZ ? F.shape[1] : 1u;
     o.rate = F.rate;
     return o;
+}
+
+/* A fluence grid in the header of a batch instance: the same fields without
+ * the window, in 60 bytes (FluenceL takes 96: a batch of 16,800 instances
+ * that fits XO_NOALLOC_SCRATCH_BYTES with these would not with those). */
+struct FluenceGrid {
+    float top_left[3];
+    float k;
+    float inv_step[3];
+    int32_t enabled;
+    float shape[3];
+    uint32_t offset;
+    uint32_t nx, ny;
+    int32_t rate;
+};
+
+inline FluenceGrid fluence_without_window(const FluenceL &F) {
+    return FluenceGrid{{F.top_left[0], F.top_left[1], F.top_left[2]}, F.k,
+                       {F.inv_step[0], F.inv_step[1], F.inv_step[2]}, F.enabled,
+                       {F.shape[0], F.shape[1], F.shape[2]}, F.offset, F.nx, F.ny, F.rate};
 }
 
 struct McmlParams {

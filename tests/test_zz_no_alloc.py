@@ -133,3 +133,34 @@ def test_noalloc_rejects_a_batch_beyond_the_scratch_array():
     finally:
         mem.close()
         b.context.close()
+
+
+def test_noalloc_fills_the_scratch_array():
+    """Per one-item instance the array holds 8 layer records of 64 bytes, a
+    header of at most 344 and a work item of 16: the most instances that fit
+    at those sizes run."""
+    align = lambda v: (v + 255) // 256 * 256  # noqa: E731
+    free = N.XO_NOALLOC_SCRATCH_BYTES - align(4 * N.XO_MAX_SEEDS) - 256
+    n = free // (512 + 344 + 16)
+    while align(512 * n) + align(344 * n) + align(16 * n) > free:
+        n -= 1
+    b = Batch(small_batch(40, seed=6, budget=(64, 65)),
+              rnginit=0x5EED000000000001)
+    arr, lut, nacc = b.pack()
+    many = (N.XoBatchInstance * n)()
+    for i in range(n):
+        many[i] = arr[i % 40]
+    mem = DeviceMemory()
+    try:
+        lut_d = mem.upload(np.asarray(lut, dtype=np.float32))
+        acc_d = mem.alloc(8 * nacc)
+        print('case', n, flush=True)
+        ref, rep_ref = b.context.run_batch(many, lut, b.opts(chunk=64), nacc)
+        rep = b.context.run_batch_noalloc(many, lut_d, len(lut),
+                                          b.opts(chunk=64), acc_d, nacc)
+        np.testing.assert_array_equal(mem.download(acc_d, nacc, np.uint64),
+                                      ref)
+        assert rep.packets == rep_ref.packets == 64 * n
+    finally:
+        mem.close()
+        b.context.close()
