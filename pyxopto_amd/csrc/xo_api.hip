@@ -880,7 +880,8 @@ static int mcml_run(xo_ctx *ctx, const xo_mcml_cfg *cfg, const float *lut, uint3
     P.lds_lut = (nlut && nlut <= XO_LDS_LUT_MAX) ? nlut : 0u;
     /* packets are inside the layers between the first and the last */
     for (uint32_t i = 1; i + 1 < cfg->num_layers; ++i)
-        P.pf_rare |= xo::pf_needs_rare(cfg->pf_kind, cfg->layers[i].pf);
+        P.pf_rare |= xo::pf_needs_rare(cfg->pf_kind, cfg->layers[i].pf,
+                                       (flags & XO_FLAG_FAST_MATH) && !trace);
     int bpc = 1;
     if (flags & XO_FLAG_STATIC_SCHEDULE) {
         const bool small = !(flags & XO_FLAG_NO_LDS_BINS) && naccum <= XO_LDS_BINS_MAX;

@@ -464,9 +464,10 @@ template <class M> __host__ __device__ inline bool pf_rare(int kind, const PfL &
              (pf.lc <= -0x1p-60f || pf.lc > 1.0f) && fabsf(pf.lc) <= 0x1p59f);
 }
 
-/* Host: pf_rare of a packed phase function, for either arithmetic. */
-inline uint32_t pf_needs_rare(int kind, const xo_pf &f) {
-    return pf_rare<MathExact>(kind, PfL{f.g, f.beta, f.a, f.b, f.c, 0u, 0u}) ? 1u : 0u;
+/* Host: pf_rare of a packed phase function in the arithmetic of a run. */
+inline uint32_t pf_needs_rare(int kind, const xo_pf &f, bool fast) {
+    const PfL pf{f.g, f.beta, f.a, f.b, f.c, 0u, 0u};
+    return (fast ? pf_rare<MathFast>(kind, pf) : pf_rare<MathExact>(kind, pf)) ? 1u : 0u;
 }
 
 /* mcsim_pf_sample_angles: returns cos(theta), the azimuth as a fraction of

@@ -107,7 +107,7 @@ struct McmlParams {
     uint32_t lds_lut;
     FluenceL fluence;      /* the grid of cfg.fluence, with its window    */
     uint32_t pf_rare;      /* some medium needs the general phase-function
-                              sampling code (xo::pf_rare)                 */
+                              sampling code (xo::pf_rare): which build runs */
 };
 
 struct McvoxParams {
