@@ -109,6 +109,8 @@ inline bool any_fluence(const BatchHdr *hdr, size_t n) {
 
 /* Items a wave of the resident grid should find in the queue at least. */
 constexpr uint64_t kItemsPerWave = 2;
+/* Items that an instance of mean size is cut into for that at most. */
+constexpr uint64_t kPiecesPerInstance = 2048;
 
 /* One work-queue item: packets [first, first + count) of one instance. */
 struct BatchItem {
