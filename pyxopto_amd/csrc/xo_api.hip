@@ -653,6 +653,7 @@ void xo_ctx_destroy(xo_ctx *ctx) {
     if (ctx->trace_data) (void)hipFree(ctx->trace_data);
     if (ctx->trace_n) (void)hipFree(ctx->trace_n);
     if (ctx->trace_stage) (void)hipHostFree(ctx->trace_stage);
+    for (uint32_t k = 0; k < ctx->free_mlp_stages; ++k) (void)hipHostFree(ctx->mlp_stages[k]);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);

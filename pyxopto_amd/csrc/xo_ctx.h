@@ -27,6 +27,12 @@
         }                                                                             \
     } while (0)
 
+namespace xo {
+/* Pinned stages of a context's networks: as many as run a small forward pass
+ * at the same time, at most this many (beyond, such a pass copies). */
+constexpr uint32_t kMaxStages = 8;
+} // namespace xo
+
 struct xo_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -60,6 +66,11 @@ struct xo_ctx {
     int32_t *trace_n = nullptr;
     size_t trace_n_cap = 0;
     float *trace_stage = nullptr; /* pinned; a trace on its way to the host */
+    /* pinned memory for small forward passes of the context's networks, not
+     * in use now, and how many there are in all */
+    float *mlp_stages[xo::kMaxStages] = {};
+    uint32_t free_mlp_stages = 0, num_mlp_stages = 0;
+    std::mutex stage_mu;
     std::mutex mu;
 };
 

@@ -1353,6 +1353,36 @@ __global__ void __launch_bounds__(WNT) train_weights_kernel(const WgArgs g) {
  * out of it: 5 % at 9900 rows. */
 constexpr uint64_t kStageBytes = 2048u * 1024u;
 
+/* A stage of the context for the time of one forward call. Making one takes
+ * 50-300 us, more than a small pass: xo_mlp_create sees to it that there is
+ * one, and the networks of a context share them. */
+struct Stage {
+    xo_ctx *ctx;
+    float *p = nullptr;
+    explicit Stage(xo_ctx *c, bool wanted) : ctx(c) {
+        if (!wanted) return;
+        std::lock_guard<std::mutex> lock(ctx->stage_mu);
+        if (ctx->free_mlp_stages) {
+            p = ctx->mlp_stages[--ctx->free_mlp_stages];
+        } else if (ctx->num_mlp_stages < xo::kMaxStages) {
+            if (hipHostMalloc((void **)&p, kStageBytes, hipHostMallocDefault) == hipSuccess) {
+                ++ctx->num_mlp_stages;
+            } else {
+                p = nullptr;
+                (void)hipGetLastError();
+            }
+        }
+    }
+    /* nothing on the device uses it any more */
+    void give_back() {
+        if (!p) return;
+        std::lock_guard<std::mutex> lock(ctx->stage_mu);
+        ctx->mlp_stages[ctx->free_mlp_stages++] = p;
+        p = nullptr;
+    }
+    Stage(const Stage &) = delete;
+};
+
 struct xo_mlp {
     xo_ctx *ctx = nullptr;
     hipStream_t stream = nullptr;
@@ -1387,8 +1417,6 @@ struct xo_mlp {
     uint16_t *zrow = nullptr;         /* zeros read for rows past a layer's width */
     float *loss_part = nullptr;       /* fused step: one partial loss per row block */
     bool fusable = false, train_fused = false, wt_dirty = true;
-    float *stage = nullptr;           /* kStageBytes of pinned memory: the rows of a small
-                                         forward pass, then their outputs */
     hipEvent_t ev0 = nullptr, ev1 = nullptr; /* around a forward pass's kernels */
     float *loss = nullptr;            /* per training step */
     uint32_t loss_cap = 0;
@@ -1796,7 +1824,6 @@ void xo_mlp_destroy(xo_mlp *N) {
             if (p) (void)hipFree(p);
     for (auto &kv : N->dw_tables)
         if (kv.second) (void)hipFree(kv.second);
-    if (N->stage) (void)hipHostFree(N->stage);
     if (N->ev0) (void)hipEventDestroy(N->ev0);
     if (N->ev1) (void)hipEventDestroy(N->ev1);
     if (N->stream) (void)hipStreamDestroy(N->stream);
@@ -1914,7 +1941,10 @@ xo_mlp *xo_mlp_create(xo_ctx *ctx, const uint32_t *dims, uint32_t nlayers, uint3
             }
             if ((e = hipMalloc(&N->wtt, 2 * tb)) != hipSuccess) return bad("allocation", e);
         }
+        Stage(ctx, true).give_back();
     }
+    if ((e = hipEventCreate(&N->ev0)) != hipSuccess) return bad("hipEventCreate", e);
+    if ((e = hipEventCreate(&N->ev1)) != hipSuccess) return bad("hipEventCreate", e);
     /* where each matrix entry's bf16 copies are: W_l [in][ld out] and
      * W_l^T [out][ld in]; biases have none */
     std::vector<uint64_t> bi(P, kNotMatrix), ti(P, kNotMatrix);
@@ -1976,31 +2006,27 @@ int xo_mlp_forward(xo_mlp *N, const float *x, uint64_t n, float *y, double *kern
     std::lock_guard<std::mutex> lock(N->mu);
     MLP_CHECK(hipSetDevice(N->ctx->device));
     const uint32_t nin = N->dims[0], nout = N->dims[N->nlayers];
-    if (!N->ev0) MLP_CHECK(hipEventCreate(&N->ev0));
-    if (!N->ev1) MLP_CHECK(hipEventCreate(&N->ev1));
-    if (N->fusable && !N->stage &&
-        hipHostMalloc((void **)&N->stage, kStageBytes, hipHostMallocDefault) != hipSuccess) {
-        N->stage = nullptr; /* copies then */
-        (void)hipGetLastError();
-    }
+    /* the outputs start on a 16-byte boundary, as in N->y */
+    auto y_start = [nin](uint64_t rows) { return (4u * rows * nin + 15u) & ~(uint64_t)15u; };
+    auto fits = [&](uint64_t rows) { return y_start(rows) + 4u * rows * nout <= kStageBytes; };
+    /* the last pass is the smallest */
+    Stage stage(N->ctx, N->fusable && n && fits((n - 1u) % N->max_batch + 1u));
     double total = 0.0;
     int rc = 0;
     if (N->fusable && N->wt_dirty && refresh_transposed(N)) rc = -1;
     for (uint64_t r = 0; r < n && rc == 0; r += N->max_batch) {
         const uint32_t B = (uint32_t)(n - r < N->max_batch ? n - r : N->max_batch);
         const uint64_t xbytes = 4ull * B * nin, ybytes = 4ull * B * nout;
-        /* the outputs start on a 16-byte boundary, as in N->y */
-        const uint64_t ystart = (xbytes + 15u) & ~(uint64_t)15u;
-        const bool staged = N->stage && ystart + ybytes <= kStageBytes;
-        float *ys = staged ? N->stage + ystart / 4u : N->y;
+        const bool staged = stage.p && fits(B);
+        float *ys = staged ? stage.p + y_start(B) / 4u : N->y;
         if (staged) {
-            std::memcpy(N->stage, x + r * nin, xbytes);
+            std::memcpy(stage.p, x + r * nin, xbytes);
         } else if (N->fusable) {
             if (hipMemcpyAsync(N->xf, x + r * nin, xbytes, hipMemcpyHostToDevice, N->stream) !=
                 hipSuccess) { rc = -1; break; }
         } else if (upload_rows(N, x + r * nin, B)) { rc = -1; break; }
         if (hipEventRecord(N->ev0, N->stream) != hipSuccess) { rc = -1; break; }
-        if (N->fusable ? forward_fused(N, B, staged ? N->stage : N->xf, ys) : forward(N, B)) {
+        if (N->fusable ? forward_fused(N, B, staged ? stage.p : N->xf, ys) : forward(N, B)) {
             rc = -1;
             break;
         }
@@ -2017,6 +2043,8 @@ int xo_mlp_forward(xo_mlp *N, const float *x, uint64_t n, float *y, double *kern
         (void)hipEventElapsedTime(&ms, N->ev0, N->ev1);
         total += ms;
     }
+    /* after a failure only once the stream is known to be done with it */
+    if (rc == 0 || hipStreamSynchronize(N->stream) == hipSuccess) stage.give_back();
     if (kernel_ms) *kernel_ms = total;
     return rc;
 }

@@ -2,6 +2,7 @@
 product of the same bf16 operands (every transpose case, ragged tiles), the
 gradient against the CPU restatement, captured training steps against
 eager ones, and what the trained network gains over Monte Carlo alone."""
+import threading
 import time
 
 import numpy as np
@@ -157,6 +158,41 @@ def test_forward_of_few_rows_equals_forward_of_many(ctx, dims):
         ys, _ = net.forward(x[lo:lo + rows])
         np.testing.assert_array_equal(ys, y[lo:lo + rows])
     net.close()
+
+
+def test_networks_of_a_context_share_the_pinned_stages(ctx):
+    """Small forward passes borrow pinned memory from the context: more
+    networks than it keeps stages, each asked from a thread of its own, give
+    what they give alone, first calls included."""
+    nets, xs, ref = [], [], []
+    rng = np.random.default_rng(5)
+    for k in range(11):
+        p = M.init_params(S.DIMS, seed=20 + k)
+        x = rng.uniform(-1, 1, (37 + 400 * k, S.DIMS[0])).astype(np.float32)
+        alone = S.Network(S.DIMS, ctx)
+        alone.set_params(p)
+        ref.append(alone.forward(x)[0])
+        alone.close()
+        net = S.Network(S.DIMS, ctx)
+        net.set_params(p)
+        nets.append(net)
+        xs.append(x)
+    wrong = []
+
+    def ask(k):
+        for _ in range(20):
+            if not np.array_equal(nets[k].forward(xs[k])[0], ref[k]):
+                wrong.append(k)
+
+    threads = [threading.Thread(target=ask, args=(k,))
+               for k in range(len(nets))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for net in nets:
+        net.close()
+    assert not wrong
 
 
 @pytest.mark.parametrize('dims', [(5, 64, 64, 10), S.DIMS, (5, 256, 100),
