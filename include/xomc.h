@@ -135,7 +135,10 @@ enum xo_run_flags {
     XO_FLAG_FAST_MATH = 1u << 3,
     /* The caller's trace_data is all zeros: the entries past a packet's last
      * event are then left as they are instead of being written. */
-    XO_FLAG_TRACE_ZEROED = 1u << 4
+    XO_FLAG_TRACE_ZEROED = 1u << 4,
+    /* Batches: work items of xo_batch_opts.chunk packets, also where a launch
+     * would leave waves without items. */
+    XO_FLAG_WHOLE_CHUNKS = 1u << 5
 };
 
 /* Phase-function parameters; the union of McPf for Hg, MHg and Lut. */
@@ -368,10 +371,11 @@ typedef struct xo_batch_instance {
 typedef struct xo_batch_opts {
     uint32_t chunk;             /* packets per work-queue item (>= 1), at most:
                                    fewer where a launch would otherwise leave
-                                   waves without items                        */
+                                   waves without items (xo_batch_chunk)       */
     uint32_t block;             /* threads per block: 64, 128 or 256          */
     uint32_t blocks_per_cu;     /* 0: as many as fit                          */
-    uint32_t flags;             /* XO_FLAG_FAST_MATH; other flags are ignored */
+    uint32_t flags;             /* XO_FLAG_FAST_MATH, XO_FLAG_WHOLE_CHUNKS;
+                                   other flags are ignored                    */
     float w_min;                /* roulette threshold for every instance     */
     float lottery_chance;
     int32_t use_lottery;
@@ -509,6 +513,12 @@ int xo_mcvox_run_trace(xo_ctx *ctx, const xo_mcvox_cfg *cfg,
                        uint64_t npackets, uint32_t lanes, uint32_t flags,
                        const xo_trace *trace, float *trace_data, int32_t *trace_n,
                        uint64_t *accum, uint64_t naccum, xo_run_report *report);
+
+/* Packets of a work item with which xo_batch_run and a plan run this batch:
+ * opts->chunk, or fewer (see xo_batch_opts). The kernel that runs, its results
+ * and what else opts say are not looked at. */
+int xo_batch_chunk(xo_ctx *ctx, const xo_batch_instance *instances, uint32_t ninstances,
+                   const xo_batch_opts *opts, uint32_t *chunk);
 
 /* Run a batch of layered-media instances in one persistent launch: a device
  * work queue of (instance, chunk of packets) items; lanes take packets of

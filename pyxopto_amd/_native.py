@@ -45,6 +45,7 @@ XO_FLAG_NO_LDS_BINS = 1 << 1
 XO_FLAG_PACKET_KEYED = 1 << 2
 XO_FLAG_FAST_MATH = 1 << 3
 XO_FLAG_TRACE_ZEROED = 1 << 4
+XO_FLAG_WHOLE_CHUNKS = 1 << 5
 (XO_MATH_LOG, XO_MATH_SIN_TURNS, XO_MATH_COS_TURNS, XO_MATH_SQRT, XO_MATH_RCP,
  XO_MATH_RSQRT, XO_MATH_CBRT, XO_MATH_EXP) = range(8)
 
@@ -254,6 +255,8 @@ PROTOTYPES = {
                                        POINTER(c_uint64), c_uint64,
                                        POINTER(c_uint64),
                                        POINTER(XoRunReport)]),
+    'xo_batch_chunk': (c_int, [c_void_p, POINTER(XoBatchInstance), c_uint32,
+                               POINTER(XoBatchOpts), POINTER(c_uint32)]),
     'xo_batch_run': (c_int, [c_void_p, POINTER(XoBatchInstance), c_uint32,
                              POINTER(c_float), c_uint32, POINTER(XoBatchOpts),
                              POINTER(c_uint64), c_uint64,
@@ -618,6 +621,15 @@ class Context:
                                  _ptr(accum, c_uint64), c_uint64(naccum),
                                  ctypes.byref(rep)), 'xo_batch_run')
         return accum, rep
+
+    def batch_chunk(self, instances, opts: XoBatchOpts) -> int:
+        """Packets of a work item with which run_batch runs this batch."""
+        chunk = c_uint32()
+        check(lib().xo_batch_chunk(self._h, instances,
+                                   c_uint32(len(instances)),
+                                   ctypes.byref(opts), ctypes.byref(chunk)),
+              'xo_batch_chunk')
+        return int(chunk.value)
 
     def batch_plan(self, instances, lut, opts: XoBatchOpts, naccum: int):
         """xo_batch_plan_create: the batch uploaded and its launch captured

@@ -350,16 +350,37 @@ void fill_report(xo_run_report *r, const unsigned long long *stats, uint32_t lan
     r->total_ms = total_ms;
 }
 
-int pack_batch(const char *fn, uint32_t waves, const xo_batch_instance *inst, uint32_t ninst, bool have_lut,
-               uint32_t nlut, const xo_batch_opts *opts, uint64_t naccum,
+bool batch_block_ok(const char *fn, const xo_batch_opts &opts) {
+    if (!opts.block || opts.block == 64 || opts.block == 128 || opts.block == 256) return true;
+    set_error("%s: block must be 64, 128 or 256 (got %u)", fn, opts.block);
+    return false;
+}
+
+uint64_t batch_chunk(const xo_batch_opts &opts, uint64_t waves, uint64_t total, uint32_t ninst) {
+    const uint64_t chunk = opts.chunk ? opts.chunk : 1024u;
+    if (!waves || (opts.flags & XO_FLAG_WHOLE_CHUNKS)) return chunk;
+    /* small enough that every resident wave finds kItemsPerWave items, down
+     * to one packet per lane (100 instances of 1e5 packets in chunks of 2048
+     * are 4900 items for 7168 waves: 9.2 ms, 5.5 in smaller ones). No
+     * smaller: a wave that runs through more instances at a time reads more
+     * layers and changes rounds more often (256 instances: 50 ms at 2 items
+     * per wave, 51 at 4, 76 at 16). And not so small that one instance is in
+     * the hands of more than kPiecesPerInstance waves: they add to the same
+     * few detector bins, and that is what then bounds it (an isotropic 1 mm
+     * slab of 1e6 packets: 4.36 ms in 64-packet items on all 7168 waves, 3.5
+     * in 1000 or 2000 pieces, 4.0 in 4000; of a medium that absorbs, 1.16,
+     * 1.11, 1.03 and 1.04). */
+    const uint64_t part =
+        std::max(total / (waves * kItemsPerWave), total / ninst / kPiecesPerInstance) / 64u * 64u;
+    return std::min<uint64_t>(chunk, std::max<uint64_t>(part, 64u));
+}
+
+int pack_batch(const char *fn, uint32_t waves, const xo_batch_instance *inst, uint32_t ninst,
+               bool have_lut, uint32_t nlut, const xo_batch_opts *opts, uint64_t naccum,
                std::vector<LayerL> &layers, std::vector<BatchHdr> &hdr,
                std::vector<BatchItem> &items, uint64_t *total, uint32_t *block_out) {
     const uint32_t block = opts->block ? opts->block : 256u;
-    if (block != 64 && block != 128 && block != 256) {
-        set_error("%s: block must be 64, 128 or 256 (got %u)", fn, block);
-        return -1;
-    }
-    const uint64_t chunk = opts->chunk ? opts->chunk : 1024u;
+    if (!batch_block_ok(fn, *opts)) return -1;
     if (opts->method != XO_METHOD_AW && opts->method != XO_METHOD_AR &&
         opts->method != XO_METHOD_MBL) {
         set_error("%s: unknown stepping method %d", fn, opts->method);
@@ -456,23 +477,7 @@ int pack_batch(const char *fn, uint32_t waves, const xo_batch_instance *inst, ui
         if (p.cls != q.cls) return p.cls < q.cls;
         return p.steps > q.steps;
     });
-    /* chunks small enough that every resident wave finds kItemsPerWave of
-     * them, down to one packet per lane (100 instances of 1e5 packets in
-     * chunks of 2048 are 4900 items for 7168 waves: 9.2 ms, 5.5 in smaller
-     * ones). No smaller: a wave that runs through more instances at a time
-     * reads more layers and changes rounds more often (256 instances: 50 ms
-     * at 2 items per wave, 51 at 4, 76 at 16). And not so small that one
-     * instance is in the hands of more than kPiecesPerInstance waves: they
-     * add to the same few detector bins, and that is what then bounds it (an
-     * isotropic 1 mm slab of 1e6 packets: 4.36 ms in 64-packet items on all
-     * 7168 waves, 3.5 in 1000 or 2000 pieces, 4.0 in 4000; of a medium that
-     * absorbs, 1.16, 1.11, 1.03 and 1.04). */
-    uint64_t part = chunk;
-    if (waves) {
-        part = std::max(*total / (waves * kItemsPerWave), *total / ninst / kPiecesPerInstance) /
-               64u * 64u;
-        part = std::min<uint64_t>(chunk, std::max<uint64_t>(part, 64u));
-    }
+    const uint64_t part = batch_chunk(*opts, waves, *total, ninst);
     /* the instances of a group in turn, each in proportion to its packets, so
      * that all are in flight at once and their bins share the adds (4
      * instances of 1e7 packets in 2752-packet items, one after the other 121
@@ -520,20 +525,21 @@ void batch_params(const xo_batch_opts &opts, BatchParams &P) {
     P.fast_math = (opts.flags & XO_FLAG_FAST_MATH) ? 1 : 0;
 }
 
-uint32_t batch_waves(xo_ctx *ctx) {
-    int bpc = 1;
-    if (hipSetDevice(ctx->device) != hipSuccess || occupancy_batch(64u, &bpc) != hipSuccess ||
-        bpc < 1)
-        bpc = 1;
-    return (uint32_t)bpc * ctx->cus;
-}
-
 int batch_grid(xo_ctx *ctx, uint32_t block, const xo_batch_opts &opts, uint32_t *blocks) {
     int bpc = 1;
     XO_HIP(occupancy_batch(block, &bpc));
     if (opts.blocks_per_cu && (int)opts.blocks_per_cu < bpc) bpc = (int)opts.blocks_per_cu;
     if (bpc < 1) bpc = 1;
     *blocks = (uint32_t)bpc * ctx->cus;
+    return 0;
+}
+
+int batch_waves(xo_ctx *ctx, const xo_batch_opts &opts, uint32_t *waves) {
+    const uint32_t block = opts.block ? opts.block : 256u;
+    uint32_t blocks = 0;
+    XO_HIP(hipSetDevice(ctx->device));
+    if (batch_grid(ctx, block, opts, &blocks)) return -1;
+    *waves = blocks * (block / 64u);
     return 0;
 }
 
@@ -1172,6 +1178,22 @@ int xo_packet_seed(uint64_t seed, uint64_t p, uint64_t *x, uint32_t *a) {
     return 0;
 }
 
+int xo_batch_chunk(xo_ctx *ctx, const xo_batch_instance *inst, uint32_t ninst,
+                   const xo_batch_opts *opts, uint32_t *chunk) {
+    xo::clear_error();
+    if (!ctx || !inst || !opts || !chunk || ninst == 0) {
+        xo::set_error("xo_batch_chunk: null or empty argument");
+        return -1;
+    }
+    uint32_t waves = 0;
+    if (!xo::batch_block_ok("xo_batch_chunk", *opts) || xo::batch_waves(ctx, *opts, &waves))
+        return -1;
+    uint64_t total = 0;
+    for (uint32_t i = 0; i < ninst; ++i) total += inst[i].npackets;
+    *chunk = (uint32_t)xo::batch_chunk(*opts, waves, total, ninst);
+    return 0;
+}
+
 int xo_batch_run(xo_ctx *ctx, const xo_batch_instance *inst, uint32_t ninst,
                  const float *lut, uint32_t nlut, const xo_batch_opts *opts,
                  uint64_t *accum, uint64_t naccum, xo_run_report *report) {
@@ -1185,9 +1207,10 @@ int xo_batch_run(xo_ctx *ctx, const xo_batch_instance *inst, uint32_t ninst,
     std::vector<xo::BatchHdr> hdr;
     std::vector<xo::BatchItem> items;
     uint64_t total = 0;
-    uint32_t block = 0;
-    if (xo::pack_batch("xo_batch_run", xo::batch_waves(ctx), inst, ninst, lut != nullptr, nlut,
-                       opts, naccum, layers, hdr, items, &total, &block))
+    uint32_t block = 0, waves = 0;
+    if (!xo::batch_block_ok("xo_batch_run", *opts) || xo::batch_waves(ctx, *opts, &waves) ||
+        xo::pack_batch("xo_batch_run", waves, inst, ninst, lut != nullptr, nlut, opts, naccum,
+                       layers, hdr, items, &total, &block))
         return -1;
 
     std::lock_guard<std::mutex> lock(ctx->mu);

@@ -89,21 +89,26 @@ double ms_since(std::chrono::steady_clock::time_point t0);
 void fill_report(xo_run_report *r, const unsigned long long *stats, uint32_t lanes,
                  float kernel_ms, double total_ms);
 
+/* Whether the block size of a batch is one of those there are (message set
+ * if not). */
+bool batch_block_ok(const char *fn, const xo_batch_opts &opts);
+/* Packets of a work item: opts.chunk, or fewer for `waves` resident waves
+ * (0: opts.chunk). */
+uint64_t batch_chunk(const xo_batch_opts &opts, uint64_t waves, uint64_t total, uint32_t ninst);
 /* Validate a batch (fn names the entry point in messages) and build its
  * device tables: layer records [instance][XO_BATCH_MAX_LAYERS], per-instance
- * headers and the work items (chunks of at most opts->chunk packets, smaller
- * ones if `waves` resident waves would find too few; 0: opts->chunk).
- * *total: packets of all instances; *block: threads per block. Returns -1
- * (message set) on error. */
-int pack_batch(const char *fn, uint32_t waves, const xo_batch_instance *inst, uint32_t ninst, bool have_lut,
-               uint32_t nlut, const xo_batch_opts *opts, uint64_t naccum,
+ * headers and the work items (batch_chunk). *total: packets of all instances;
+ * *block: threads per block. Returns -1 (message set) on error. */
+int pack_batch(const char *fn, uint32_t waves, const xo_batch_instance *inst, uint32_t ninst,
+               bool have_lut, uint32_t nlut, const xo_batch_opts *opts, uint64_t naccum,
                std::vector<LayerL> &layers, std::vector<BatchHdr> &hdr,
                std::vector<BatchItem> &items, uint64_t *total, uint32_t *block);
 /* The launch options of a batch as kernel parameters (buffers left null). */
 void batch_params(const xo_batch_opts &opts, BatchParams &P);
-/* Blocks of the persistent batch grid for this block size and options. */
-uint32_t batch_waves(xo_ctx *ctx);
+/* Blocks of the persistent batch grid for this block size and options, and
+ * its waves (the device is made current). */
 int batch_grid(xo_ctx *ctx, uint32_t block, const xo_batch_opts &opts, uint32_t *blocks);
+int batch_waves(xo_ctx *ctx, const xo_batch_opts &opts, uint32_t *waves);
 
 /* Device layout of a voxel grid: uint8 material indices in 4x4x4 bricks of
  * 64 bytes, bricks in [z][y][x] order, voxel (x, y, z) at byte

@@ -124,9 +124,11 @@ xo_batch_plan *xo_batch_plan_create(xo_ctx *ctx, const xo_batch_instance *inst,
     xo_batch_plan *p = new xo_batch_plan();
     p->ctx = ctx;
     p->naccum = naccum;
-    if (xo::pack_batch("xo_batch_plan_create", xo::batch_waves(ctx), inst, ninst,
-                       lut != nullptr, nlut, opts, naccum, layers, hdr, items, &p->total,
-                       &p->block)) {
+    uint32_t waves = 0;
+    if (!xo::batch_block_ok("xo_batch_plan_create", *opts) ||
+        xo::batch_waves(ctx, *opts, &waves) ||
+        xo::pack_batch("xo_batch_plan_create", waves, inst, ninst, lut != nullptr, nlut, opts,
+                       naccum, layers, hdr, items, &p->total, &p->block)) {
         delete p;
         return nullptr;
     }

@@ -5,6 +5,7 @@ captured plan and alone."""
 import numpy as np
 import pytest
 
+from pyxopto_amd import _native as N
 from pyxopto_amd.mcml import batch as mbatch
 from pyxopto_amd.mcml import mc
 
@@ -51,3 +52,32 @@ def test_every_packet_runs_once(name):
     assert int(rep.packets) == total
     np.testing.assert_array_equal(acc, ref)
     b.context.close()
+
+
+def test_item_size_follows_the_grid():
+    """Items of at most the chunk, two for each wave of the grid that these
+    options launch, at least 64 packets; the whole chunk if asked for; the
+    results are those of any size."""
+    insts = [_instance(k, 40000 + k) for k in range(30)]
+    b = mbatch.Batch(insts, rnginit=XINIT)
+    arr, lut, naccum = b.pack()
+    ctx, total = b.context, sum(i.nphotons for i in insts)
+    ref, rep = ctx.run_batch(arr, lut, b.opts(), naccum)
+    for block, bpc in ((64, 0), (64, 1), (128, 3), (256, 0), (256, 1)):
+        for chunk in (50, 2048, 1 << 20):
+            print('case', block, bpc, chunk, flush=True)
+            o = b.opts(chunk=chunk, block=block, blocks_per_cu=bpc)
+            acc, rep = ctx.run_batch(arr, lut, o, naccum)
+            np.testing.assert_array_equal(acc, ref)
+            waves = int(rep.lanes) // 64
+            if bpc:
+                assert waves == bpc * block // 64 * ctx.compute_units
+            assert ctx.batch_chunk(arr, o) == min(
+                chunk, max(total // (2 * waves) // 64 * 64, 64))
+            o.flags |= N.XO_FLAG_WHOLE_CHUNKS
+            assert ctx.batch_chunk(arr, o) == chunk
+            acc, _ = ctx.run_batch(arr, lut, o, naccum)
+            np.testing.assert_array_equal(acc, ref)
+    with pytest.raises(RuntimeError, match='block must be'):
+        ctx.batch_chunk(arr, b.opts(block=96))
+    ctx.close()
