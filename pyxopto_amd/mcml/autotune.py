@@ -1,13 +1,17 @@
 """Launch-shape autotuner of the batched engine.
 
 Tunables: packets per work-queue item (chunk), threads per block and blocks
-per CU (persistent grid). Budgets are never scaled down: a wave keeps the
-instance of its item for a whole chunk, so the coherence a chunk buys
-depends on how it compares with an instance's budget. Instead, each
-candidate runs two calibration batches of instances drawn evenly from the
-batch with their full budgets (about 1e8 and 2e8 packets); the time of a
-launch is modelled as packets / rate + tail, where the tail (waves finishing
-their last items) depends on the chunk but not on the batch size. The two
+per CU (persistent grid). A launch cuts a candidate's chunk down where waves
+would be left without items (xo_batch_chunk); candidates that come to the
+same launch of the batch count once, under the chunk that it uses. Budgets
+are never scaled down: a wave keeps the instance of its item for a whole
+chunk, so the coherence a chunk buys depends on how it compares with an
+instance's budget. Instead, each candidate runs two calibration batches of
+instances drawn evenly from the batch with their full budgets (about 1e8 and
+2e8 packets), both in the items that the whole batch gets
+(XO_FLAG_WHOLE_CHUNKS); the time of a launch is modelled as packets / rate +
+tail, where the tail (waves finishing their last items) depends on the chunk
+but not on the batch size. The two
 runs give rate and tail, the model predicts the whole batch, and the
 candidate with the shortest predicted time wins. A plain "fastest
 calibration run" would pick chunks far too small: the tail weighs much
@@ -28,6 +32,9 @@ CANDIDATES = [(chunk, block, bpc)
               for block in (64, 256)
               for bpc in (0,)]
 CACHE = os.path.join(N.DATA_DIR, 'autotune.json')
+# part of a cache key: entries tuned with another item order or other item
+# sizes are not used
+VERSION = 2
 CALIBRATION_PACKETS = 200_000_000
 VERIFY_PACKETS = 2_000_000_000
 
@@ -77,13 +84,14 @@ def _packets(arr) -> int:
 
 def sweep(ctx, arr, lut, naccum, base_opts, candidates=CANDIDATES):
     """[(predicted_ms, chunk, block, bpc, rate_packets_per_ms, tail_ms)] for
-    every candidate, best first."""
+    every launch that the candidates come to, best first; chunk is the one
+    that the whole batch is run in."""
     big = calibration_batch(arr)
     small = (N.XoBatchInstance * ((len(big) + 1) // 2))()
     for j in range(len(small)):
         small[j] = big[2 * j]
     w1, w2, wf = _packets(small), _packets(big), _packets(arr)
-    res = []
+    res, seen = [], set()
     for chunk, block, bpc in candidates:
         o = N.XoBatchOpts()
         o.chunk, o.block, o.blocks_per_cu = chunk, block, bpc
@@ -91,6 +99,11 @@ def sweep(ctx, arr, lut, naccum, base_opts, candidates=CANDIDATES):
         o.use_lottery = base_opts.use_lottery
         o.method = base_opts.method
         o.flags = base_opts.flags
+        o.chunk = chunk = ctx.batch_chunk(arr, o)
+        if (chunk, block, bpc) in seen:
+            continue
+        seen.add((chunk, block, bpc))
+        o.flags |= N.XO_FLAG_WHOLE_CHUNKS
         _, r1 = ctx.run_batch(small, lut, o, naccum)
         _, r2 = ctx.run_batch(big, lut, o, naccum)
         t1, t2 = r1.kernel_ms, r2.kernel_ms
@@ -109,8 +122,9 @@ def tuned_opts(batch, packed, force: bool = False):
     arr, lut, naccum = packed
     ctx = batch.context
     base = batch.opts()
-    key = '{}cu-{}{}'.format(ctx.compute_units, _signature(arr),
-                             '-fast' if base.flags & N.XO_FLAG_FAST_MATH else '')
+    key = '{}cu-{}{}-v{}'.format(
+        ctx.compute_units, _signature(arr),
+        '-fast' if base.flags & N.XO_FLAG_FAST_MATH else '', VERSION)
     cache = _load_cache()
     if not force and key in cache:
         chunk, block, bpc = cache[key]['best']
