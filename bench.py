@@ -463,21 +463,19 @@ def timed(step, steps: int, warmup: int):
     return reps, time.perf_counter() - t0
 
 
-def roofline(reps, voxel: bool, workload: str, ceil=None):
+def roofline(reps, voxel: bool, workload: str):
     kernel_s = sum(r.kernel_ms for r in reps) * 1e-3
     achieved = sum(algorithmic_slots(r, voxel) for r in reps) / kernel_s / 1e12
     out = {'bound': 'valu', 'achieved': achieved, 'peak': PEAK_SLOTS / 1e12,
            'unit': 'T lane-op slots/s', 'frac': achieved / (PEAK_SLOTS / 1e12),
            'traffic': TRAFFIC_BYTES_PER_LAUNCH.get(workload)}
-    if voxel and ceil:
-        dep = sum(r.deposits for r in reps)
-        out['atomic_deposits_per_s'] = dep / kernel_s
-        out['atomic_GBps'] = dep * 8 / kernel_s / 1e9
-        out['atomic_frac_of_probe'] = dep / kernel_s / ceil['atomic_u64_per_s']
+    if voxel:
+        # LDS adds and cached ones among them: no share of the atomic rate
+        out['deposits_per_s'] = sum(r.deposits for r in reps) / kernel_s
     return out
 
 
-def config_leg(name: str, steps: int, warmup: int, ceil, cpu: bool,
+def config_leg(name: str, steps: int, warmup: int, cpu: bool,
                cpu_packets: int):
     """One single-simulation configuration timed on its own: packets/s,
     steps/s, its roofline and its CPU baseline."""
@@ -493,7 +491,7 @@ def config_leg(name: str, steps: int, warmup: int, ceil, cpu: bool,
            'kernel_ms_per_step': kernel_s / steps * 1e3,
            'transport_steps_per_s': sum(r.steps for r in reps) / wall,
            'lanes': int(reps[-1].lanes),
-           'roofline': roofline(reps, voxel, name, ceil)}
+           'roofline': roofline(reps, voxel, name)}
     if voxel:
         out['voxel_crossings_per_s'] = sum(r.voxel_crossings
                                            for r in reps) / kernel_s
@@ -585,13 +583,11 @@ def main():
         'kernel_ms_per_step': kernel_s / args.steps * 1e3,
     }
     ceil = ceilings(sim.context)
-    out['roofline'] = roofline(reps, voxel, config['workload'], ceil)
+    out['roofline'] = roofline(reps, voxel, config['workload'])
     out['roofline']['hbm_copy_GBps'] = ceil['copy_GBps']
     out['measured_ceilings'] = ceil
     if voxel:
-        for key in ('atomic_deposits_per_s', 'atomic_GBps',
-                    'atomic_frac_of_probe'):
-            out[key] = out['roofline'][key]
+        out['deposits_per_s'] = out['roofline']['deposits_per_s']
         out['voxel_crossings_per_s'] = sum(r.voxel_crossings
                                            for r in reps) / kernel_s
     if hasattr(sim, 'bench_upload_inclusive'):
@@ -602,9 +598,9 @@ def main():
         out['batched_vs_plain'] = value / plain['packets_per_s']
     if hasattr(sim, 'bench_insts') and not args.no_legs:
         out['configs'] = {
-            'slab_1mm': config_leg('slab_1mm', 20, 3, ceil,
+            'slab_1mm': config_leg('slab_1mm', 20, 3,
                                    not args.no_cpu_baseline, 1_000_000),
-            'skin_vessel_200': config_leg('skin_vessel_200', 3, 1, ceil,
+            'skin_vessel_200': config_leg('skin_vessel_200', 3, 1,
                                           not args.no_cpu_baseline,
                                           1_000_000)}
     if hasattr(sim, 'bench_insts') and not args.no_published:

@@ -335,7 +335,9 @@ typedef struct xo_run_report {
     uint64_t steps;             /* iterations of the transport loop           */
     uint64_t boundary_steps;    /* of which ended on a boundary               */
     uint64_t voxel_crossings;   /* mcvox: voxel faces crossed (incl. steps)   */
-    uint64_t deposits;          /* fluence deposits issued                    */
+    uint64_t deposits;          /* non-zero fluence deposits (more than the
+                                   atomic adds in memory: several may have
+                                   been added up in LDS before)               */
     uint64_t truncated;         /* packets stopped at XO_MAX_PACKET_STEPS     */
     uint32_t lanes;             /* lanes launched                             */
     uint32_t threads_used;      /* lanes that ran >= 1 packet (num_kernels)   */
@@ -444,8 +446,11 @@ typedef struct xo_ctx xo_ctx;
 xo_ctx *xo_ctx_create(int device, uint32_t max_lanes, uint64_t xinit);
 void xo_ctx_destroy(xo_ctx *ctx);
 
-/* Lanes the device runs concurrently for the transport kernels (the
- * persistent grid size) and the context's seed capacity. */
+/* Lanes the device runs concurrently for the layered kernel (the persistent
+ * grid of a run without a fluence grid, exact arithmetic; it follows the
+ * kernel's registers and may differ between versions of this library, unlike
+ * the default lane count of static-schedule runs) and the context's seed
+ * capacity. */
 int xo_ctx_info(xo_ctx *ctx, uint32_t *persistent_lanes, uint32_t *max_lanes,
                 uint32_t *compute_units);
 
@@ -732,7 +737,10 @@ uint64_t xo_mlp_param_count(xo_mlp *mlp);
 /* Set (and reset the optimizer state) / read the fp32 parameters. */
 int xo_mlp_set_params(xo_mlp *mlp, const float *params, uint64_t n);
 int xo_mlp_get_params(xo_mlp *mlp, float *params, uint64_t n);
-/* y[n][dims[nlayers]] = network(x[n][dims[0]]); kernel_ms may be NULL. */
+/* y[n][dims[nlayers]] = network(x[n][dims[0]]). kernel_ms (may be NULL): time
+ * of the kernels; where the kernel itself reads the rows from and writes the
+ * outputs to host memory (passes of up to 2 MiB of both), the way over the
+ * bus is part of it. */
 int xo_mlp_forward(xo_mlp *mlp, const float *x, uint64_t n, float *y, double *kernel_ms);
 /* Mean squared error of one batch (n <= max_batch rows) and its gradient
  * with respect to every parameter (packed like the parameters). */

@@ -21,7 +21,8 @@ enum {
     XO_STAT_PACKETS = 2,   /* packets launched                           */
     XO_STAT_THREADS = 3,   /* lanes that launched at least one packet    */
     XO_STAT_CROSSINGS = 4, /* mcvox: voxel faces crossed                 */
-    XO_STAT_DEPOSITS = 5,  /* fluence atomics issued                     */
+    XO_STAT_DEPOSITS = 5,  /* non-zero fluence deposits: adds in LDS, in a
+                              lane's cache or in memory                  */
     XO_STAT_TRUNCATED = 6, /* packets stopped at XO_MAX_PACKET_STEPS     */
     XO_STAT_COUNT = 7
 };
