@@ -454,6 +454,11 @@ void xo_ctx_destroy(xo_ctx *ctx);
 int xo_ctx_info(xo_ctx *ctx, uint32_t *persistent_lanes, uint32_t *max_lanes,
                 uint32_t *compute_units);
 
+/* How the last xo_mcml_run or xo_mcvox_run (or a traced one) of the context
+ * was launched: threads per block, blocks, and the fluence bins that each
+ * block held in LDS (0: none). For tests and measurements. */
+int xo_ctx_last_launch(xo_ctx *ctx, uint32_t *block, uint32_t *blocks, uint32_t *window_bins);
+
 /* Copy the mutable RNG state x of the first n lanes to the host
  * (Mc.run(copyseeds=True), xopto/mcml/mc.py:962-966) or overwrite it. */
 int xo_ctx_get_rng(xo_ctx *ctx, uint32_t n, uint64_t *x_out, uint32_t *a_out);

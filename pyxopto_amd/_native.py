@@ -228,6 +228,8 @@ PROTOTYPES = {
     'xo_ctx_destroy': (None, [c_void_p]),
     'xo_ctx_info': (c_int, [c_void_p, POINTER(c_uint32), POINTER(c_uint32),
                             POINTER(c_uint32)]),
+    'xo_ctx_last_launch': (c_int, [c_void_p, POINTER(c_uint32),
+                                   POINTER(c_uint32), POINTER(c_uint32)]),
     'xo_ctx_get_rng': (c_int, [c_void_p, c_uint32, POINTER(c_uint64),
                                POINTER(c_uint32)]),
     'xo_ctx_set_rng': (c_int, [c_void_p, c_uint32, POINTER(c_uint64),
@@ -534,6 +536,14 @@ class Context:
             self.close()
         except Exception:
             pass
+
+    def last_launch(self):
+        """(threads per block, blocks, fluence bins held in LDS) of the last
+        layered or voxel run."""
+        v = [c_uint32() for _ in range(3)]
+        check(lib().xo_ctx_last_launch(self._h, *map(ctypes.byref, v)),
+              'xo_ctx_last_launch')
+        return tuple(int(x.value) for x in v)
 
     def get_rng(self, n: int):
         x = np.empty(n, dtype=np.uint64)

@@ -203,6 +203,9 @@ static int shape_launch(xo_ctx *ctx, const xo_fluence &F, const float src[3], in
         }
     }
     *blocks = (P.lanes + *block - 1) / *block;
+    ctx->last_block = *block;
+    ctx->last_blocks = *blocks;
+    ctx->last_window = P.fluence.bins;
     return 0;
 }
 
@@ -681,6 +684,18 @@ int xo_ctx_info(xo_ctx *ctx, uint32_t *persistent_lanes, uint32_t *max_lanes,
     if (persistent_lanes) *persistent_lanes = choose_lanes(ctx, 0, bpc, ~0ull);
     if (max_lanes) *max_lanes = ctx->max_lanes;
     if (compute_units) *compute_units = ctx->cus;
+    return 0;
+}
+
+int xo_ctx_last_launch(xo_ctx *ctx, uint32_t *block, uint32_t *blocks, uint32_t *window_bins) {
+    if (!ctx) {
+        xo::set_error("null context");
+        return -1;
+    }
+    std::lock_guard<std::mutex> lock(ctx->mu);
+    if (block) *block = ctx->last_block;
+    if (blocks) *blocks = ctx->last_blocks;
+    if (window_bins) *window_bins = ctx->last_window;
     return 0;
 }
 

@@ -39,6 +39,9 @@ struct xo_ctx {
     uint32_t max_lanes = 0;
     uint32_t cus = 0;
     uint32_t lds_per_cu = 65536;
+    /* launch of the last single-simulation run: threads per block, blocks,
+     * fluence bins that each block held in LDS */
+    uint32_t last_block = 0, last_blocks = 0, last_window = 0;
     uint64_t *rng_x = nullptr;
     uint32_t *rng_a = nullptr;
     unsigned long long *counters = nullptr; /* [0] packet counter, [1..] stats */
