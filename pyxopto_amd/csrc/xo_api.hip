@@ -167,7 +167,7 @@ FluenceL fluence_window(const xo_fluence &F, const float src[3], uint32_t budget
  * waves land on SIMDs that are full). 6e6 packets into an 8000-bin r-z grid,
  * hardware arithmetic: 176 ms with every deposit in memory, 26 ms with 2025
  * bins in seven blocks of 256, 18.5 with 4096 in four of 384, 9.5 with all
- * 8000 in two of 768. A lane count that the caller left open (`open`) is cut
+ * 8000 in two of 768 (the transport step as it was then; 8.2 now). A lane count that the caller left open (`open`) is cut
  * to what is resident. */
 template <class Params, class Fit>
 static int shape_launch(xo_ctx *ctx, const xo_fluence &F, const float src[3], int waves,

@@ -93,7 +93,7 @@ batch_kernel(const BatchParams P) {
      * truncated packets and, with fluence grids, deposits), added with LDS
      * atomics, and the simulation sphere of its packet (source position and
      * squared radius), read only where some packet of the wave has a finite
-     * one: kept in registers they would take eight of the loop's 64 */
+     * one: kept in registers they would take eight of the loop's 72 */
     extern __shared__ __attribute__((aligned(16))) uint32_t smem[];
     constexpr uint32_t kCounts = FLU ? 5 : 4;
     const uint32_t nthreads = blockDim.x;
@@ -124,8 +124,9 @@ batch_kernel(const BatchParams P) {
     uint32_t pkt_steps = 0;
     /* the per-step fields of the packet's current layer (layer_state):
      * read again only when the layer may change (a new packet, a boundary
-     * event), not in every step (+14 % packets/s; the compiler spills a
-     * few rarely used registers to stay at 64) */
+     * event), not in every step (+14 % packets/s). At 72 registers the
+     * compiler spills rarely used ones: 1-2 in the hardware arithmetic, 8
+     * in the exact one, 7-31 in builds with fluence grids */
     float4 lt = make_float4(0.f, 0.f, 0.f, 0.f);
     LanePf lpf{0.f, 0.f, 0.f, 0u, 0u};
     auto layer_of = [&](int32_t l) -> const LayerL & {

@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(64 * kWaves) sv_kernel(const SvParams P) {
                 /* sva_next_voxel, :130-152 */
                 const int32_t nx = (int32_t)(dist[0] <= dist[1]) & (int32_t)(dist[0] <= dist[2]);
                 const int32_t ny =
-                    !nx & (int32_t)(dist[1] <= dist[0]) & (int32_t)(dist[1] <= dist[2]);
+                    (nx ^ 1) & (int32_t)(dist[1] <= dist[0]) & (int32_t)(dist[1] <= dist[2]);
                 const int32_t nz = !(nx | ny);
                 v[0] += e1.d[0] < 0.0f ? -nx : nx;
                 v[1] += e1.d[1] < 0.0f ? -ny : ny;
