@@ -40,12 +40,11 @@ SERVING_QPS = 250.0                     # requests/s of the serving run
 # WRITE_SIZE of one launch, each scaled by what the counter reads for a
 # 1 GiB device-to-device copy (profiles/batch_kernel_layered_batch_4096.md,
 # profiles/mcvox_kernel_skin_vessel_200.md,
-# profiles/mcml_kernel_slab_1mm_and_surrogate.md). Offline figures: measured
-# with the builds that those profiles name, hardware arithmetic; a larger fluence
-# window has since taken some of skin_vessel_200's atomics into LDS.
-TRAFFIC_BYTES_PER_LAUNCH = {'layered_batch_4096': 2.585e11,
-                            'skin_vessel_200': 7.52e11,
-                            'slab_1mm': 5.3e6}
+# profiles/mcml_kernel_slab_1mm_and_surrogate.md). Offline figures of the
+# kernels as they are in this tree, hardware arithmetic.
+TRAFFIC_BYTES_PER_LAUNCH = {'layered_batch_4096': 2.883e11,
+                            'skin_vessel_200': 7.43e11,
+                            'slab_1mm': 5.2e6}
 
 METRIC = ('photon packets/s (1 GPU) batched vs plain; p50/p99 solve latency '
           'at fixed QPS')
