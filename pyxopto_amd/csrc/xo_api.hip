@@ -501,7 +501,9 @@ int pack_batch(const char *fn, uint32_t waves, const xo_batch_instance *inst, ui
             set_error("%s: too many work items; raise the chunk size", fn);
             return -1;
         }
-        const uint64_t turns = pieces / turn + 1u;
+        /* at most about four million steps of this loop (10 ms) a group */
+        const uint64_t turns =
+            std::min<uint64_t>(pieces / turn, (4u << 20) / (uint64_t)(end - i)) + 1u;
         for (size_t k = i; k < end; ++k) order[k].due = turns - 1u; /* all in the first */
         for (uint64_t t = 0; t < turns; ++t)
             for (size_t k = i; k < end; ++k) {
